@@ -58,8 +58,6 @@ constexpr int kNW = kWG / kWave;           // waves per workgroup
 constexpr int kMaxChunks = 128;            // vocab <= 262144
 constexpr int kMaxVocab = kMaxChunks * kChunk;
 constexpr int kRowCap = 2048;              // LDS entries per row in the finaliser
-constexpr int kRadixBits = 10;
-constexpr int kBins = 1 << kRadixBits;     // radix digits per round
 constexpr int kMaxLevel = 31;              // candidate levels: e >= 2^-L, L in [0, 31]
 constexpr int64_t kMaxRows = 65536;
 constexpr int64_t kMaxSpecBatch = 16384;
@@ -68,7 +66,7 @@ constexpr uint32_t kNone = 0xffffffffu;
 enum Mode : int { kModeSpec = 0, kModeSample = 1, kModeDense = 2 };
 // kChunkPenCands: penalised candidates follow the others, in no particular order
 enum ChunkFlag : uint32_t { kChunkOverflow = 1u, kChunkHasTok = 2u, kChunkPenCands = 4u };
-enum RowFlag : uint32_t { kRowFiltered = 1u, kRowList = 2u, kRowEmpty = 4u, kRowSlow = 8u, kRowRefilled = 16u };
+enum RowFlag : uint32_t { kRowFiltered = 1u, kRowList = 2u, kRowEmpty = 4u, kRowRefilled = 8u };
 
 // Per-chunk result of the streaming pass.
 struct ChunkRec {
@@ -1500,390 +1498,753 @@ __device__ __forceinline__ void select_entries(FS& f, uint32_t mask, const uint6
   }
 }
 
-// Passes over a whole row for the slow path: fn(index, x) for every element,
-// 16-byte vectors spread over the workgroup.
-template <int DT, typename Fn>
-__device__ __forceinline__ void row_pass(const Params& p, const char* rowp, const uint32_t* bm, int64_t i0, int64_t i1,
-                                         Fn fn) {
+// ---------------------------------------------------------------------------
+// Whole-row passes: rows whose support is not among their candidates
+// ---------------------------------------------------------------------------
+constexpr int kQueue = kHash / kFNW;  // words of LDS (the draft hash's) a wave queues logits in
+
+// A logit no element with p >= v lies below (slack for the roundings of p's
+// exponent, polynomial and division: together under 2^-16 octaves).
+__device__ __forceinline__ float x_floor(const RowK& K, float v) {
+  if (!(v > 0.0f)) return -__builtin_inff();
+  const double t = log2(static_cast<double>(v) * static_cast<double>(K.s)) - 1.0e-3;
+  const float x = static_cast<float>((t + static_cast<double>(K.mcmax)) / K.cd);
+  return -next_up(-x);
+}
+
+// A logit no element with p < v lies above.
+__device__ __forceinline__ float x_ceil(const RowK& K, float v) {
+  const double t = log2(static_cast<double>(v) * static_cast<double>(K.s)) + 1.0e-3;
+  return next_up(static_cast<float>((t + static_cast<double>(K.mcmax)) / K.cd));
+}
+
+// Orders a wave's own LDS traffic (the LDS serves a wave in order; this keeps
+// the compiler from moving it).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// What travels with a queued logit: nothing, the second row's logit at the
+// same index, or the index.
+enum Beside : int { kAlone = 0, kPairX = 1, kIndex = 2 };
+
+// Chunk j of a row as one wave loads it: vector u of lane t (words 4 u .. of
+// its registers) is the chunk's vector 64 u + t (lanes past the chunk's end
+// re-read its last vector). The passes below loop over a chunk's elements a
+// few at a time with a uniform register index, not unrolled over the 32 of a
+// lane: the same time, and a third of the code.
+typedef uint32_t u32x32 __attribute__((ext_vector_type(32)));
+typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
+template <int DT>
+struct ChunkRegs {
+  using type = u32x16;
+};
+template <>
+struct ChunkRegs<F32> {
+  using type = u32x32;
+};
+template <int DT>
+struct ChunkData {
+  static constexpr int kVecs = kChunk / (kWave * Elem<DT>::kPerVec);
+  typename ChunkRegs<DT>::type d;
+};
+
+template <int DT>
+__device__ __forceinline__ void load_chunk(const Params& p, const char* rowp, int j, ChunkData<DT>& c) {
   constexpr int EPV = Elem<DT>::kPerVec;
-  const u32x4* src = reinterpret_cast<const u32x4*>(rowp);
-  for (int64_t v = i0 / EPV + threadIdx.x; v < i1 / EPV; v += kFW) {
-    const u32x4 d = src[v];
-    uint32_t word = bm ? bm[(v * EPV) >> 5] : 0u;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int c0 = j * kChunk;
+  const int nvc = (p.vocab - c0 < kChunk ? p.vocab - c0 : kChunk) / EPV;
+  const u32x4* src = reinterpret_cast<const u32x4*>(rowp) + c0 / EPV;
 #pragma unroll
-    for (int e = 0; e < EPV; ++e) {
-      const int64_t i = v * EPV + e;
-      float x = vec_elem<DT>(d, e);
-      if (bm && ((word >> (i & 31)) & 1u)) x = penalise(x, p.pen);
-      fn(i, x);
-    }
+  for (int u = 0; u < ChunkData<DT>::kVecs; ++u) {
+    const int v = u * kWave + lane;
+    const u32x4 x = src[v < nvc ? v : nvc - 1];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) c.d[4 * u + k] = x[k];
   }
 }
 
-// Whole-row exact cutoff by three radix passes over the row (slow path). With
-// kCount every element weighs 1 instead of fx46(p): thr = k then gives the
-// k-th largest p (duplicates counted) and *mass the count at and above it.
-template <int DT, bool kCount = false, class FS>
-__device__ __forceinline__ bool select_row(const Params& p, FS& f, int row, const RowK& K, uint64_t thr, float* cut, uint64_t* mass) {
-  const int t = threadIdx.x;
-  const char* rowp = row_ptr(p, row);
-  const uint32_t* bm = row_bitmap(p, row);
-  uint64_t* bins = f.u.bins[0];
-  uint32_t prefix = 0;
-  uint64_t above = 0;
-  constexpr int kPer = kBins / kFW;
-  for (int round = 0; round < 3; ++round) {
-    const int shift = 20 - round * kRadixBits;
+// kStep elements of a lane from a chunk's registers, processed: elements
+// kStep * st .. of the lane's 32, whose chunk index is *i0 onwards.
+template <int DT, int kStep>
+__device__ __forceinline__ void chunk_step(const Params& p, const ChunkData<DT>& c, const uint32_t* bm, int j, int st,
+                                           float (&x)[kStep], int* i0) {
+  constexpr int EPV = Elem<DT>::kPerVec;
+  constexpr int kPerWord = EPV / 4;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int u = st * kStep / EPV, e0 = st * kStep % EPV;
+  const int i = (u * kWave + lane) * EPV + e0;
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) bins[kPer * t + q] = 0;
-    __syncthreads();
-    row_pass<DT>(p, rowp, bm, 0, p.vocab, [&](int64_t, float x) {
-      const uint32_t b = __float_as_uint(pval(K, x));
-      if ((b >> (shift + kRadixBits)) == prefix)
-        __hip_atomic_fetch_add(&bins[(b >> shift) & (kBins - 1)], kCount ? uint64_t{1} : fx46(__uint_as_float(b)),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    });
-    __syncthreads();
-    const int g0 = kPer * (kFW - 1 - t);
-    uint64_t own = 0;
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) own += bins[g0 + q];
-    uint64_t tot;
-    const uint64_t incl = block_incl_scan(own, f.red[round & 1], &tot);
-    const uint64_t need = thr > above ? thr - above : 0;
-    if (tot < need) {
-      // the row holds less than thr: the reference clamps to the last sorted
-      // value, the row minimum, and keeps everything
-      if (round != 0) return false;  // cannot happen: later rounds include the crossing
-      float mn = __builtin_inff();
-      row_pass<DT>(p, rowp, bm, 0, p.vocab, [&](int64_t, float x) {
-        const float v = pval(K, x);
-        mn = v < mn ? v : mn;
-      });
-      uint64_t key = static_cast<uint64_t>(__float_as_uint(mn));
-      key = ~block_max_u64<kFW>(~key, f.red[2]);  // min via max of complements
-      __syncthreads();
-      *cut = __uint_as_float(static_cast<uint32_t>(key));
-      *mass = tot;
-      return true;
+  for (int w = 0; w < kStep / kPerWord; ++w) {
+    const uint32_t word = c.d[st * (kStep / kPerWord) + w];
+    if constexpr (DT == F32) {
+      x[w] = __uint_as_float(word);
+    } else {
+      x[2 * w] = bits_to_float<DT>(word & 0xffffu);
+      x[2 * w + 1] = bits_to_float<DT>(word >> 16);
     }
-    if (incl >= need && incl - own < need) {
-      uint64_t acc = incl - own;
-      int d = g0;
-      for (int q = kPer - 1; q >= 0; --q) {
-        const uint64_t bq = bins[g0 + q];
-        if (acc + bq >= need) {
-          d = g0 + q;
-          break;
-        }
-        acc += bq;
+  }
+  if (bm) {
+    const int at = j * kChunk + i;
+    const uint32_t pb = at < p.vocab ? bm[at >> 5] >> (at & 31) : 0u;
+#pragma unroll
+    for (int e = 0; e < kStep; ++e) x[e] = (pb >> e) & 1u ? penalise(x[e], p.pen) : x[e];
+  }
+  *i0 = i;
+}
+
+// What fn of a pass gets at a time: kBatch queued logits per lane, so that
+// the exact p of several are under way together (two waves per SIMD do not
+// hide the latency of one's dependent chain).
+template <int kBeside>
+struct Batch {
+  static constexpr int kN = kBeside == kAlone ? 4 : 2;
+  float x[kN];
+  uint32_t beside[kN];
+  bool valid[kN];
+};
+
+// One wave over loaded chunk j of a row: fn(batch) on the elements whose
+// processed logit lies in [lo, hi] (a NaN counts as inside), in no particular
+// order. fn evaluates p exactly (some 32 instructions, in binary64), and a pass
+// wants few of the elements, so each element's test only appends it to the
+// wave's queue in LDS and fn runs on full waves of queued ones. The chunk's
+// elements are all done on return.
+template <int DT, int kBeside, typename Fn>
+__device__ __forceinline__ void chunk_pass(const Params& p, const ChunkData<DT>& c, const ChunkData<DT>& c1,
+                                           const uint32_t* bm, int j, float lo, float hi, uint32_t* q, Fn fn) {
+  using B = Batch<kBeside>;
+  constexpr int kWords = kBeside == kAlone ? 1 : 2;
+  constexpr int kStep = kBeside == kAlone ? 4 : 2;  // elements between drains
+  static_assert((kStep + B::kN) * kWave * kWords <= kQueue, "queue size");
+  const int lane = threadIdx.x & (kWave - 1);
+  const int nel = p.vocab - j * kChunk < kChunk ? p.vocab - j * kChunk : kChunk;
+  uint32_t n = 0;  // queued (wave-uniform)
+#pragma unroll 1
+  for (int st = 0; st < 32 / kStep; ++st) {
+    float x[kStep], x1[kStep];
+    int i0;
+    chunk_step<DT, kStep>(p, c, bm, j, st, x, &i0);
+    if constexpr (kBeside == kPairX) chunk_step<DT, kStep>(p, c1, bm, j, st, x1, &i0);
+    const bool in_row = i0 < nel;
+#pragma unroll
+    for (int e = 0; e < kStep; ++e) {
+      const bool in = in_row && !(x[e] < lo) && !(x[e] > hi);
+      const uint64_t m = __ballot(in);
+      if (in) {
+        const uint32_t at = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), n)) * kWords;
+        q[at] = __float_as_uint(x[e]);
+        if constexpr (kBeside == kPairX) q[at + 1] = __float_as_uint(x1[e]);
+        if constexpr (kBeside == kIndex) q[at + 1] = static_cast<uint32_t>(j * kChunk + i0 + e);
       }
-      f.sel[0] = static_cast<uint32_t>(d);
-      f.sel64[0][0] = above + acc;
-      f.sel64[0][1] = bins[d];
+      n += static_cast<uint32_t>(__builtin_popcountll(m));
     }
-    __syncthreads();
-    const uint32_t d = f.sel[0];
-    above = f.sel64[0][0];
-    prefix = (prefix << kRadixBits) | d;
-    if (round == 2) {
-      *cut = __uint_as_float(prefix);
-      *mass = above + f.sel64[0][1];
+    wave_lds_fence();
+    // whole batches; after the last step also the rest
+    const uint32_t most = st == 32 / kStep - 1 ? 0u : B::kN * kWave - 1;
+#pragma unroll 1
+    while (n > most) {
+      const uint32_t take = n < static_cast<uint32_t>(B::kN * kWave) ? n : static_cast<uint32_t>(B::kN * kWave);
+      n -= take;
+      B b;
+#pragma unroll
+      for (int k = 0; k < B::kN; ++k) {
+        const uint32_t i = static_cast<uint32_t>(k * kWave + lane);
+        b.valid[k] = i < take;
+        const uint32_t at = (n + (b.valid[k] ? i : 0u)) * kWords;
+        b.x[k] = __uint_as_float(q[at]);
+        b.beside[k] = kWords > 1 ? q[at + kWords - 1] : 0u;
+      }
+      wave_lds_fence();
+      fn(b);
     }
   }
-  __syncthreads();
-  return true;
 }
 
-// Appends the elements of chunk j with p >= cut to slot s's entries, in
-// index order, as the chunk's new range. Returns false if they do not fit.
+// The chunk's registers hold their loads' results from here on (otherwise the
+// compiler waits for the loads of the next chunk too wherever this one is read).
+template <int DT>
+__device__ __forceinline__ void chunk_arrived(ChunkData<DT>& c) {
+  asm volatile("" : "+v"(c.d));
+}
+
+// each(j, chunk, chunk1) over every chunk of a row (kPair: and of a second
+// row), wave w on chunks w, w + kFNW, ... With one workgroup per CU the next
+// chunk's loads are in flight while a chunk is worked on; with two the other
+// waves cover them.
+template <int DT, bool kPair, class FS, typename Each>
+__device__ __forceinline__ void each_chunk(const Params& p, const char* row0, const char* row1, Each each) {
+  constexpr bool kAhead = FS::kBits > 10;
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  ChunkData<DT> c, c1, next, next1;
+  if (w < p.nch) {
+    load_chunk<DT>(p, row0, w, c);
+    if constexpr (kPair) load_chunk<DT>(p, row1, w, c1);
+  }
+#pragma unroll 1
+  for (int j = w; j < p.nch; j += kFNW) {
+    if constexpr (!kAhead) {
+      if (j > w) {
+        load_chunk<DT>(p, row0, j, c);
+        if constexpr (kPair) load_chunk<DT>(p, row1, j, c1);
+      }
+    }
+    chunk_arrived<DT>(c);
+    if constexpr (kPair) chunk_arrived<DT>(c1);
+    if constexpr (kAhead) {
+      if (j + kFNW < p.nch) {
+        load_chunk<DT>(p, row0, j + kFNW, next);
+        if constexpr (kPair) load_chunk<DT>(p, row1, j + kFNW, next1);
+      }
+    }
+    each(j, c, c1);
+    if constexpr (kAhead) {
+      c = next;
+      if constexpr (kPair) c1 = next1;
+    }
+  }
+}
+
+template <class FS>
+__device__ __forceinline__ uint32_t* wave_queue(FS& f) {
+  return f.hash + __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave) * kQueue;
+}
+
+// chunk_pass over every chunk of a row.
+template <int DT, class FS, typename Fn>
+__device__ __forceinline__ void row_pass(const Params& p, FS& f, int row, float lo, float hi, Fn fn) {
+  const uint32_t* bm = row_bitmap(p, row);
+  uint32_t* q = wave_queue(f);
+  each_chunk<DT, false, FS>(p, row_ptr(p, row), nullptr, [&](int j, const ChunkData<DT>& c, const ChunkData<DT>&) {
+    chunk_pass<DT, kAlone>(p, c, c, bm, j, lo, hi, q, fn);
+  });
+}
+
+// The smallest processed logit of a row (a NaN, whose p is 0, as -inf), per lane.
 template <int DT, class FS>
-__device__ __forceinline__ bool refill_chunk(const Params& p, FS& f, int s, int row, const RowK& K, int j, float cut) {
-  constexpr int EPV = Elem<DT>::kPerVec;
-  // elements per thread, contiguous, whole vectors (threads past the chunk idle)
-  constexpr int EPT = kChunk / kFW > EPV ? kChunk / kFW : EPV;
-  const int t = threadIdx.x;
-  const char* rowp = row_ptr(p, row);
+__device__ __forceinline__ float lane_row_min(const Params& p, int row) {
+  constexpr int kStep = 4;
   const uint32_t* bm = row_bitmap(p, row);
-  const int64_t c0 = static_cast<int64_t>(j) * kChunk;
-  const int64_t nel = p.vocab - c0 < kChunk ? p.vocab - c0 : kChunk;
-  const int64_t mine = t * EPT < kChunk ? nel : 0;  // this thread's elements lie below c0 + mine
-  float pv[EPT];
-  uint32_t keep = 0;
+  float mn = __builtin_inff();
+  each_chunk<DT, false, FS>(p, row_ptr(p, row), nullptr, [&](int j, const ChunkData<DT>& c, const ChunkData<DT>&) {
+#pragma unroll 1
+    for (int st = 0; st < 32 / kStep; ++st) {
+      float x[kStep];
+      int i0;
+      chunk_step<DT, kStep>(p, c, bm, j, st, x, &i0);
+      if (j * kChunk + i0 >= p.vocab) continue;
 #pragma unroll
-  for (int q = 0; q < EPT / EPV; ++q) {
-    const int64_t i0 = c0 + static_cast<int64_t>(t) * EPT + q * EPV;
-    u32x4 d{0, 0, 0, 0};
-    if (i0 < c0 + mine) d = reinterpret_cast<const u32x4*>(rowp)[i0 / EPV];
-    const uint32_t word = (bm && i0 < c0 + mine) ? bm[i0 >> 5] : 0u;
+      for (int e = 0; e < kStep; ++e) mn = x[e] != x[e] ? -__builtin_inff() : (x[e] < mn ? x[e] : mn);
+    }
+  });
+  return mn;
+}
+
+// Slot s's list entries 0 .. n - 1 selected for `thr` (kCount: by counts).
+template <bool kCount, class FS>
+__device__ __forceinline__ bool select_list(FS& f, int s, uint32_t n, uint64_t thr, float* cut, uint64_t* mass) {
+  uint32_t eb[2][kEPT];
+  uint64_t ew[2][kEPT];
 #pragma unroll
-    for (int e = 0; e < EPV; ++e) {
-      const int64_t i = i0 + e;
-      float v = 0.0f;
-      if (i < c0 + mine) {
-        float x = vec_elem<DT>(d, e);
-        if (bm && ((word >> (i & 31)) & 1u)) x = penalise(x, p.pen);
-        v = pval(K, x);
-      }
-      pv[q * EPV + e] = v;
-      if (i < c0 + mine && v >= cut) keep |= 1u << (q * EPV + e);
+  for (int s1 = 0; s1 < 2; ++s1) {
+#pragma unroll
+    for (int q = 0; q < kEPT; ++q) {
+      const uint32_t e = static_cast<uint32_t>(threadIdx.x + kFW * q);
+      const bool in = s1 == s && e < n;
+      eb[s1][q] = in ? f.ent[s].pbits[e] : 0u;
+      ew[s1][q] = !in ? 0u : (kCount ? 1u : fx46(__uint_as_float(eb[s1][q])));
     }
   }
-  const uint32_t own = static_cast<uint32_t>(__builtin_popcount(keep));
-  uint64_t tot;
-  const uint64_t incl = block_incl_scan(own, f.red[0], &tot);
-  const uint32_t base = f.aux[s].n;
-  if (base + tot > static_cast<uint64_t>(kRowCap)) {
+  const uint64_t t2[2] = {thr, thr};
+  float c1[2];
+  uint64_t m1[2];
+  bool o1[2], set1[2];
+  __syncthreads();  // every lane has read the list and its count
+  select_entries<false>(f, 1u << s, t2, eb, ew, false, c1, m1, o1, set1);
+  *cut = s == 0 ? c1[0] : c1[1];
+  *mass = s == 0 ? m1[0] : m1[1];
+  return s == 0 ? o1[0] : o1[1];
+}
+
+// Lanes with `hit` append b to slot s's list (entries past kRowCap are counted
+// only); e: the entry's index in the vocabulary, stored with kIndexed.
+template <bool kIndexed, class FS>
+__device__ __forceinline__ void list_append(FS& f, int s, uint32_t* count, bool hit, uint32_t b, uint32_t e) {
+  const uint64_t m = __ballot(hit);
+  if (m == 0) return;
+  uint32_t at = 0;
+  if ((threadIdx.x & (kWave - 1)) == 0)
+    at = __hip_atomic_fetch_add(count, static_cast<uint32_t>(__builtin_popcountll(m)), __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_WORKGROUP);
+  at = lane_bcast_u32(at, 0) + lanes_below(m);
+  if (hit && at < static_cast<uint32_t>(kRowCap)) {
+    f.ent[s].pbits[at] = b;
+    if constexpr (kIndexed) f.ent[s].eidx[at] = e;
+  }
+}
+
+// The largest bin (searching down from the top) at which the bins' sum reaches
+// need: its index and the sum above it and in it; false when the total is less.
+// Ends with a barrier. bins: kFW * kPer values.
+template <int kPer, class FS>
+__device__ __forceinline__ bool crossing_bin(FS& f, const uint64_t* bins, uint64_t need, uint64_t* red, uint32_t* bin,
+                                             uint64_t* above, uint64_t* in, uint64_t* total) {
+  const int g0 = kPer * (kFW - 1 - static_cast<int>(threadIdx.x));
+  uint64_t own = 0;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) own += bins[g0 + q];
+  const uint64_t incl = block_incl_scan(own, red, total);
+  if (*total < need) {
     __syncthreads();
     return false;
   }
-  uint32_t pos = base + static_cast<uint32_t>(incl) - own;
+  if (incl >= need && incl - own < need) {
+    uint64_t acc = incl - own;
+    int d = g0;
 #pragma unroll
-  for (int i = 0; i < EPT; ++i) {
-    if ((keep >> i) & 1u) {
-      f.ent[s].pbits[pos] = __float_as_uint(pv[i]);
-      f.ent[s].eidx[pos] = static_cast<uint32_t>(c0 + static_cast<int64_t>(t) * EPT + i);
-      ++pos;
+    for (int q = kPer - 1; q >= 0; --q) {
+      const uint64_t bq = bins[g0 + q];
+      if (acc + bq >= need) {
+        d = g0 + q;
+        break;
+      }
+      acc += bq;
     }
-  }
-  // the chunk's old entries drop out of the select (p = 0 cannot reach the cutoff)
-  const uint32_t os = f.cstart[s][j], oc = f.ccount[s][j];
-  for (uint32_t e = os + t; e < os + oc; e += kFW) f.ent[s].pbits[e] = 0u;
-  __syncthreads();
-  if (t == 0) {
-    f.cstart[s][j] = base;
-    f.ccount[s][j] = static_cast<uint32_t>(tot);
-    f.plain[s][j] = 1;
-    f.aux[s].n = base + static_cast<uint32_t>(tot);
-    f.bound[s][j] = 0.0f;
+    f.sel[0] = static_cast<uint32_t>(d);
+    f.sel64[0][0] = acc;
+    f.sel64[0][1] = bins[d];
   }
   __syncthreads();
+  *bin = f.sel[0];
+  *above = f.sel64[0][0];
+  *in = f.sel64[0][1];
   return true;
 }
 
-// Collects the whole support {p >= cut} of a row into slot s's entries,
-// chunk by chunk (slow path); false if it does not fit.
+// A whole row's cutoff in two passes, the usual way for a support beyond the
+// LDS entries. The first bins approximate masses (hardware exp2 of the exponent
+// in units of 2^-31, 1/16 octave per bin; binary32 LDS atomics took four times
+// as long as integer ones) of the elements p >= v_min and finds the bin where
+// they reach thr; the second, over the elements of the
+// bins beside it and above, forms the exact mass above those bins and gathers
+// theirs, which decide the cutoff exactly. The first pass only chooses the
+// window: it is checked against the exact masses, and false is returned (the
+// exact digit rounds of select_row follow) when the cutoff is not inside or the
+// window holds more than the list.
+constexpr int kWinShift = 19;                                      // bits of a float above 4 mantissa bits
+constexpr int kWinBins = 2 * kFW;                                  // 64 octaves
+constexpr int kWinBase = (0x4f000000 >> kWinShift) - kWinBins + 16;  // bin 0; p = 1 (2^31 units) lies below the top 16
+
 template <int DT, class FS>
-__device__ __forceinline__ bool collect_support(const Params& p, FS& f, int s, int row, const RowK& K, float cut) {
-  if (threadIdx.x == 0) f.aux[s].n = 0;
+__device__ __forceinline__ bool select_window(const Params& p, FS& f, int s, int row, const RowK& K, uint64_t thr,
+                                              float v_min, float* cut, uint64_t* mass) {
+  constexpr int kStep = 4;
+  const int t = threadIdx.x;
+  uint32_t* fb = reinterpret_cast<uint32_t*>(f.u.bins[1]);
+  uint64_t* bins = f.u.bins[0];
+  const float inf = __builtin_inff();
+  __syncthreads();  // earlier reads of the bins and of the list
+#pragma unroll
+  for (int q = 0; q < 2; ++q) fb[2 * t + q] = 0u;
+  if (t == 0) f.gcount[s] = 0;
   __syncthreads();
-  for (int j = 0; j < p.nch; ++j) {
-    if (threadIdx.x == 0) {
-      f.cstart[s][j] = f.aux[s].n;
-      f.ccount[s][j] = 0;
-    }
-    __syncthreads();
-    if (!refill_chunk<DT>(p, f, s, row, K, j, cut)) return false;
+  {
+    const uint32_t* bm = row_bitmap(p, row);
+    const float lo = x_floor(K, v_min);
+    // exponents of p in units of 2^-31
+    const float c = p.c, nm = 31.0f - K.mcmax - __builtin_amdgcn_logf(K.s);
+    each_chunk<DT, false, FS>(p, row_ptr(p, row), nullptr, [&](int j, const ChunkData<DT>& cd, const ChunkData<DT>&) {
+#pragma unroll 1
+      for (int st = 0; st < 32 / kStep; ++st) {
+        float x[kStep];
+        int i0;
+        chunk_step<DT, kStep>(p, cd, bm, j, st, x, &i0);
+        const float lo_in = j * kChunk + i0 < p.vocab ? lo : inf;
+#pragma unroll
+        for (int e = 0; e < kStep; ++e) {
+          if (x[e] >= lo_in) {
+            const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], c, nm));
+            int b = static_cast<int>(__float_as_uint(w) >> kWinShift) - kWinBase;
+            b = b < 0 ? 0 : (b > kWinBins - 1 ? kWinBins - 1 : b);
+            __hip_atomic_fetch_add(&fb[b], static_cast<uint32_t>(w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          }
+        }
+      }
+    });
   }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+    bins[2 * t + q] = static_cast<uint64_t>(fb[2 * t + q]) << (kFxBits - 31);
+  __syncthreads();
+  uint32_t d;
+  uint64_t above, in, tot;
+  if (!crossing_bin<2>(f, bins, thr, f.red[0], &d, &above, &in, &tot)) return false;
+  if (d < 2u || d > static_cast<uint32_t>(kWinBins - 3)) return false;
+  const float v_lo = __uint_as_float((d - 1u + kWinBase) << kWinShift) * 0x1p-31f;
+  const float v_hi = __uint_as_float((d + 2u + kWinBase) << kWinShift) * 0x1p-31f;
+  uint64_t own = 0;
+  row_pass<DT>(p, f, row, x_floor(K, v_lo), inf, [&](const Batch<kAlone>& b) {
+    float v[b.kN];
+#pragma unroll
+    for (int k = 0; k < b.kN; ++k) {
+      v[k] = pval(K, b.x[k]);
+      own += b.valid[k] && v[k] >= v_hi ? fx46(v[k]) : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < b.kN; ++k)
+      list_append<false>(f, s, &f.gcount[s], b.valid[k] && v[k] >= v_lo && v[k] < v_hi, __float_as_uint(v[k]), 0u);
+  });
+  const uint64_t hi = block_sum(own, f.red[1]);
+  const uint32_t n = f.gcount[s];  // every append precedes the sum's barrier
+  if (hi >= thr || n > static_cast<uint32_t>(kRowCap)) return false;
+  uint64_t m;
+  if (!select_list<false>(f, s, n, thr - hi, cut, &m)) return false;
+  *mass = hi + m;
   return true;
 }
 
-// Resolves the cutoffs of the unit's nr rows: list mode (kRowList: the support
+// Exact cutoff of a whole row: c = max{v : sum over the row's p >= v of
+// fx46(p) >= thr} (kCount: every element weighs 1, so thr = k gives the k-th
+// largest p, duplicates counted), *mass the sum at and above it. v_min: a p the
+// cutoff probably does not lie below. Masses take select_window's two passes
+// first. What those leave undecided, and counts, take radix rounds on the bits
+// of p as in select_entries: a pass over the row bins the masses of the current
+// digit, the crossing digit's elements are gathered by a second pass into slot
+// s's entries and finished by select_entries when they fit, else the next digit
+// is binned. A row that holds less than thr in all keeps everything (the
+// reference clamps to the last sorted value, the row minimum). The draft hash
+// and slot s's entries are overwritten.
+template <int DT, bool kCount, class FS>
+__device__ __forceinline__ void select_row(const Params& p, FS& f, int s, int row, const RowK& K, uint64_t thr,
+                                           float v_min, float* cut, uint64_t* mass) {
+  const int t = threadIdx.x;
+  if constexpr (!kCount) {
+    if (select_window<DT>(p, f, s, row, K, thr, v_min, cut, mass)) return;
+  }
+  uint64_t* bins = f.u.bins[0];
+  const float inf = __builtin_inff();
+  float lo = -inf, hi = inf;
+  uint32_t prefix = 0;
+  uint64_t above = 0;
+#pragma unroll 1
+  for (int round = 0; round < 3; ++round) {
+    const int shift = round == 0 ? 30 - FS::kBits : (round == 1 ? 30 - 2 * FS::kBits : 0);
+    const int width = round == 2 ? 30 - 2 * FS::kBits : FS::kBits;
+    __syncthreads();  // earlier reads of the bins and of the list
+#pragma unroll
+    for (int q = 0; q < FS::kPer; ++q) bins[FS::kPer * t + q] = 0;
+    if (t == 0) f.gcount[s] = 0;
+    __syncthreads();
+    row_pass<DT>(p, f, row, lo, hi, [&](const Batch<kAlone>& b) {
+#pragma unroll
+      for (int k = 0; k < b.kN; ++k) {
+        const uint32_t v = __float_as_uint(pval(K, b.x[k]));
+        const uint64_t w = kCount ? uint64_t{1} : fx46(__uint_as_float(v));
+        if (b.valid[k] && w && (v >> (shift + width)) == prefix)
+          __hip_atomic_fetch_add(&bins[(v >> shift) & ((1u << width) - 1u)], w, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+    });
+    __syncthreads();
+    uint32_t d;
+    uint64_t ab, in, tot;
+    if (!crossing_bin<FS::kPer>(f, bins, thr - above, f.red[round & 1], &d, &ab, &in, &tot)) {
+      // the row holds less than thr (only in the first round)
+      const float mn = -block_max_f32<kFW>(-lane_row_min<DT, FS>(p, row), reinterpret_cast<float*>(f.red[2]));
+      *cut = pval(K, mn);
+      *mass = tot;
+      return;
+    }
+    prefix = (prefix << width) | d;
+    above += ab;
+    if (round == 2) {
+      *cut = __uint_as_float(prefix);
+      *mass = above + in;
+      return;
+    }
+    // the crossing digit's elements (p from prefix << shift up to the next digit)
+    lo = prefix ? x_floor(K, __uint_as_float(prefix << shift)) : -inf;
+    hi = x_ceil(K, __uint_as_float((prefix + 1u) << shift));
+    row_pass<DT>(p, f, row, lo, hi, [&](const Batch<kAlone>& b) {
+#pragma unroll
+      for (int k = 0; k < b.kN; ++k) {
+        const uint32_t v = __float_as_uint(pval(K, b.x[k]));
+        list_append<false>(f, s, &f.gcount[s],
+                           b.valid[k] && (v >> shift) == prefix && (kCount || fx46(__uint_as_float(v)) != 0), v, 0u);
+      }
+    });
+    __syncthreads();
+    const uint32_t n = f.gcount[s];
+    if (n <= static_cast<uint32_t>(kRowCap)) {
+      uint64_t m;
+      select_list<kCount>(f, s, n, thr - above, cut, &m);
+      *mass = above + m;
+      return;
+    }
+  }
+}
+
+// Appends the elements p >= c of the chunks whose non-candidates may reach c
+// to slot s's entries, in no order, in place of those chunks' candidates
+// (whose p becomes 0). False when they do not fit. Uses the draft hash's LDS.
+template <int DT, class FS>
+__device__ __forceinline__ bool refill_chunks(const Params& p, FS& f, int s, int row, const RowK& K, float c) {
+  const int t = threadIdx.x, lane = t & (kWave - 1);
+  const int w = __builtin_amdgcn_readfirstlane(t / kWave);
+  const char* rowp = row_ptr(p, row);
+  const uint32_t* bm = row_bitmap(p, row);
+  const float lo = x_floor(K, c);
+  uint32_t* q = wave_queue(f);
+  // the chunks to re-read (lane l's bounds are chunk l's and chunk 64 + l's),
+  // dealt to the waves in turn
+  uint64_t need[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int j = h * kWave + lane;
+    need[h] = __ballot(j < p.nch && f.bound[s][j < p.nch ? j : 0] >= c);
+  }
+  int turn = 0;
+#pragma unroll 1
+  while (need[0] | need[1]) {
+    const int h = need[0] ? 0 : 1;
+    const int j = h * kWave + __builtin_ctzll(h ? need[1] : need[0]);
+    if (h) need[1] &= need[1] - 1; else need[0] &= need[0] - 1;
+    if ((turn++ & (kFNW - 1)) != w) continue;
+    ChunkData<DT> cd;
+    load_chunk<DT>(p, rowp, j, cd);
+    const uint32_t e0 = f.cstart[s][j], e1 = e0 + f.ccount[s][j];
+    for (uint32_t e = e0 + lane; e < e1; e += kWave) f.ent[s].pbits[e] = 0u;
+    chunk_pass<DT, kIndex>(p, cd, cd, bm, j, lo, __builtin_inff(), q, [&](const Batch<kIndex>& b) {
+      float v[b.kN];
+#pragma unroll
+      for (int k = 0; k < b.kN; ++k) v[k] = pval(K, b.x[k]);
+#pragma unroll
+      for (int k = 0; k < b.kN; ++k)
+        list_append<true>(f, s, &f.aux[s].n, b.valid[k] && v[k] >= c, __float_as_uint(v[k]), b.beside[k]);
+    });
+  }
+  __syncthreads();
+  return f.aux[s].n <= static_cast<uint32_t>(kRowCap);
+}
+
+// A p the top-p cutoff of a row probably does not lie below: every element
+// below it together holds less than half of 1 - top_p.
+__device__ __forceinline__ float cutoff_guess(const Params& p, uint64_t thr) {
+  const float rest = static_cast<float>(kFxOne - static_cast<double>(thr)) * static_cast<float>(1.0 / kFxOne);
+  return rest > 0.0f ? 0.5f * rest / static_cast<float>(p.vocab) : 0.0f;
+}
+
+// A resolved row's state (one thread).
+__device__ __forceinline__ void store_row(RowAux& a, uint32_t flags, float cut, uint64_t mass) {
+  a.flags = flags;
+  a.cut = cut;
+  a.mass_fx = mass;
+  a.mass_f = mass_to_f32(mass);
+}
+
+// Resolves the cutoffs of the unit's rows: list mode (kRowList: the support
 // is in the LDS entries) or dense (the support is {p >= cut} of the whole
 // row). The rows in `mask` are filtered (thr: their thresholds); their first
 // selects share their rounds, over the entries in eb / ew, whose first-round
-// masses are in the bins already. Unfiltered rows keep row_setup's state.
-template <int DT, class FS>
-__device__ __forceinline__ void resolve_rows(const Params& p, FS& f, int nr, const int (&rows)[2], const RowK (&K)[2],
-                                            uint32_t mask, const uint64_t (&thr)[2], const uint32_t (&eb)[2][kEPT],
-                                            const uint64_t (&ew)[2][kEPT]) {
+// masses are in the bins already with `hist`. Unfiltered rows keep row_setup's
+// state. A select over the entries is the row's when its cutoff lies above
+// every chunk's non-candidate bound. Otherwise that cutoff, when the entries
+// hold thr, is a lower bound of the row's: the chunks whose bound reaches it
+// are re-read (kRefill) and the entries selected again; a row they do not fit,
+// or whose entries hold less than thr, is selected whole.
+template <int DT, bool kRefill, class FS>
+__device__ __forceinline__ void resolve_rows(const Params& p, FS& f, const int (&rows)[2], const RowK (&K)[2], uint32_t mask,
+                                            const uint64_t (&thr)[2], const uint32_t (&eb)[2][kEPT],
+                                            const uint64_t (&ew)[2][kEPT], bool hist) {
   float cut[2] = {0.0f, 0.0f};
   uint64_t mass[2] = {0u, 0u};
   bool ok[2] = {false, false}, set[2] = {false, false};
-  if (mask) select_entries(f, mask, thr, eb, ew, true, cut, mass, ok, set);
-  bool generic = false;  // a row whose state thread 0 stores below
-  uint32_t flags[2] = {f.aux[0].flags & kRowEmpty, f.aux[1].flags & kRowEmpty};
+  if (!mask) return;
+  select_entries(f, mask, thr, eb, ew, hist, cut, mass, ok, set);
+  uint32_t late = 0, whole = 0;  // list rows not stored yet; rows to select whole
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     if (!((mask >> s) & 1u)) continue;  // unfiltered: P = p over the whole row
-    flags[s] = kRowFiltered | kRowList;
-    if (ok[s] && !(cut[s] > f.aux[s].bmax)) {
-      // re-read the chunks whose non-candidates may reach the cutoff
-      flags[s] |= kRowRefilled;
-      for (int j = 0; j < p.nch && ok[s]; ++j) {
-        if (f.bound[s][j] >= cut[s]) ok[s] = refill_chunk<DT>(p, f, s, rows[s], K[s], j, cut[s]);
-      }
-      if (ok[s]) {
-        uint32_t eb1[2][kEPT];
-        uint64_t ew1[2][kEPT];
-        const uint32_t n = f.aux[s].n;
-#pragma unroll
-        for (int s1 = 0; s1 < 2; ++s1) {
-#pragma unroll
-          for (int q = 0; q < kEPT; ++q) {
-            const uint32_t e = static_cast<uint32_t>(threadIdx.x + kFW * q);
-            eb1[s1][q] = (s1 == s && e < n) ? f.ent[s].pbits[e] : 0u;
-            ew1[s1][q] = fx46(__uint_as_float(eb1[s1][q]));
-          }
-        }
-        float c1[2];
-        uint64_t m1[2];
-        bool o1[2], set1[2];
-        select_entries(f, 1u << s, thr, eb1, ew1, false, c1, m1, o1, set1);
-        ok[s] = o1[s];
-        cut[s] = c1[s];
-        mass[s] = m1[s];
-      }
+    if (!ok[s] || !(cut[s] > f.aux[s].bmax)) {
+      whole |= 1u << s;
+    } else if (!set[s]) {
+      late |= 1u << s;
     }
-    if (!ok[s]) {
-      flags[s] = kRowFiltered | kRowSlow;
-      select_row<DT>(p, f, rows[s], K[s], thr[s], &cut[s], &mass[s]);
-      if (collect_support<DT>(p, f, s, rows[s], K[s], cut[s])) flags[s] |= kRowList;
-    }
-    if (flags[s] != (kRowFiltered | kRowList) || !set[s]) generic = true;
   }
-  if (generic) {
-    __syncthreads();  // every read of the rows' state above precedes the stores
-    if (threadIdx.x == 0) {
+  if (!(late | whole)) return;
+  __syncthreads();  // every read of the rows' state above precedes the stores
+  if (threadIdx.x == 0) {
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        if (s >= nr || !((mask >> s) & 1u)) continue;
-        RowAux& a = f.aux[s];
-        a.flags = flags[s];
-        a.cut = cut[s];
-        a.mass_fx = mass[s];
-        a.mass_f = mass_to_f32(mass[s]);
-      }
+    for (int s = 0; s < 2; ++s) {
+      if ((late >> s) & 1u) store_row(f.aux[s], kRowFiltered | kRowList, cut[s], mass[s]);
+    }
+  }
+  const float g0 = ok[0] ? cut[0] : cutoff_guess(p, thr[0]), g1 = ok[1] ? cut[1] : cutoff_guess(p, thr[1]);
+#pragma unroll 1
+  for (int s = 0; s < 2; ++s) {
+    if (!((whole >> s) & 1u)) continue;
+    const int row = s == 0 ? rows[0] : rows[1];
+    const RowK Ks = s == 0 ? K[0] : K[1];
+    const uint64_t th = s == 0 ? thr[0] : thr[1];
+    const float g = s == 0 ? g0 : g1;
+    float c;
+    uint64_t m;
+    uint32_t flags = kRowFiltered;
+    if (kRefill && (s == 0 ? ok[0] : ok[1]) && refill_chunks<DT>(p, f, s, row, Ks, g) &&
+        select_list<false>(f, s, f.aux[s].n, th, &c, &m)) {
+      flags |= kRowList | kRowRefilled;
+    } else {
+      select_row<DT, false>(p, f, s, row, Ks, th, g, &c, &m);
     }
     __syncthreads();
+    if (threadIdx.x == 0) store_row(f.aux[s], flags, c, m);
   }
+  // the draft hash is empty again (its LDS held the waves' queues)
+  for (int h = threadIdx.x; h < kHash; h += kFW) f.hash[h] = 0u;
+  __syncthreads();
 }
 
-// sum_{p >= c[s]} fx46(p) over the entries of the slots in `mask` (dead
-// entries hold p = 0), both slots in one block reduction.
+// sum_{p >= c[s]} fx46(p) over the entries of the slots in `mask`, both slots
+// in one block reduction.
 template <class FS>
-__device__ __forceinline__ void entries_mass2(FS& f, uint32_t mask, const float (&c)[2], uint64_t (&out)[2]) {
+__device__ __forceinline__ void entries_mass2(FS& f, uint32_t mask, const float (&c)[2], const uint32_t (&eb)[2][kEPT],
+                                              const uint64_t (&ew)[2][kEPT], uint64_t (&out)[2]) {
   uint64_t own[2] = {0u, 0u};
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     if (!((mask >> s) & 1u)) continue;
-    const uint32_t n = f.aux[s].n;
-    for (uint32_t e = threadIdx.x; e < n; e += kFW) {
-      const float v = __uint_as_float(f.ent[s].pbits[e]);
-      if (v >= c[s]) own[s] += fx46(v);
-    }
+#pragma unroll
+    for (int q = 0; q < kEPT; ++q) own[s] += __uint_as_float(eb[s][q]) >= c[s] ? ew[s][q] : 0u;
   }
   block_sum2(own[0], own[1], f.red[2], &out[0], &out[1]);
   __syncthreads();
 }
 
-// sum_{p >= c} fx46(p) over a whole row (slow path).
+// sum_{p >= c} fx46(p) over a whole row.
 template <int DT, class FS>
 __device__ __forceinline__ uint64_t row_mass(const Params& p, FS& f, int row, const RowK& K, float c) {
   uint64_t own = 0;
-  row_pass<DT>(p, row_ptr(p, row), row_bitmap(p, row), 0, p.vocab, [&](int64_t, float x) {
-    const float v = pval(K, x);
-    if (v >= c) own += fx46(v);
+  row_pass<DT>(p, f, row, x_floor(K, c), __builtin_inff(), [&](const Batch<kAlone>& b) {
+#pragma unroll
+    for (int k = 0; k < b.kN; ++k) {
+      const float v = pval(K, b.x[k]);
+      own += b.valid[k] && v >= c ? fx46(v) : 0u;
+    }
   });
   const uint64_t tot = block_sum(own, f.red[2]);
   __syncthreads();
   return tot;
 }
 
-// Top-k of the unit's rows (1 <= p.top_k < V), after their top-p cutoffs are
-// resolved: the cutoff becomes max(k-th largest p, top-p cutoff) -- the joint
-// rule of distributions.py:72-86, or the k-th largest alone when top_p = 1 --
-// with ties kept and one renormalisation over {p >= cutoff}. The k-th largest
-// is found by one select by counts over the LDS entries of both rows (ck').
-// Joint: every element that is not an entry lies below the top-p cutoff c_p
-// (its chunk's bound is, or the chunk was re-read at c_p), so ck' >= c_p
-// means the k largest are entries (ck = ck'), and ck' < c_p (or fewer than k
-// entries) means ck < c_p: the cutoff is max(ck', c_p) either way. Top-k
-// alone: the non-entries lie at or below the largest chunk bound, so ck'
-// above it is the row's; otherwise the whole row is selected by counts (slow
-// path), as is a joint row whose support exceeded the LDS entries.
+// Cutoffs of the unit's rows with top-k (1 <= p.top_k < V): max(k-th largest
+// p, top-p cutoff) -- the joint rule of distributions.py:72-86, or the k-th
+// largest alone for the rows not in `mask` (top_p = 1) -- with ties kept and
+// one renormalisation over {p >= cutoff}. The k-th largest ck of the entries
+// comes first, by a select by counts over both rows. Above every chunk's
+// non-candidate bound it is the row's, and every element at or above it is an
+// entry, so the top-p cutoff cp is decided there too: the entries' mass at and
+// above ck falls short of thr exactly when cp < ck (the cutoff is ck), and
+// otherwise cp >= ck is the entries' own. So a row whose top-p support is far
+// larger than its candidates needs no pass over the row when its k largest are
+// among them (one sequence, k = 4, V = 32000, T 0.8, top_p 0.95, top_k 50: the
+// finaliser took 25 to 164 us with top-p resolved first). Rows whose k largest
+// are not all candidates take their top-p cutoff first: a list-mode row's other
+// elements lie below cp, so its cutoff is max(ck, cp) over the entries; any
+// other row is selected by counts over the whole row.
 template <int DT, class FS>
-__device__ __forceinline__ void apply_top_k(const Params& p, FS& f, int nr, const int (&rows)[2], const RowK (&K)[2]) {
+__device__ __forceinline__ void resolve_top_k(const Params& p, FS& f, int nr, const int (&rows)[2], const RowK (&K)[2],
+                                              uint32_t mask, const uint64_t (&thr)[2], const uint32_t (&eb)[2][kEPT],
+                                              const uint64_t (&ew)[2][kEPT]) {
   const uint64_t kk = static_cast<uint64_t>(p.top_k);
-  uint32_t fl[2], lmask = 0;
-  float cp[2], bmax[2];
+  uint32_t rmask = 0;  // rows with any mass
+  float bmax[2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    fl[s] = s < nr ? f.aux[s].flags : kRowEmpty;
-    cp[s] = (fl[s] & kRowFiltered) ? f.aux[s].cut : 0.0f;
+    if (s < nr && !(f.aux[s].flags & kRowEmpty)) rmask |= 1u << s;
     bmax[s] = f.aux[s].bmax;
-    if (!(fl[s] & kRowEmpty) && (!(fl[s] & kRowFiltered) || (fl[s] & kRowList))) lmask |= 1u << s;
   }
-  if ((fl[0] & kRowEmpty) && (fl[1] & kRowEmpty)) return;
-  float ck[2] = {0.0f, 0.0f};
-  bool okk[2] = {false, false};
-  if (lmask) {
-    uint32_t eb1[2][kEPT];
-    uint64_t ew1[2][kEPT];
+  if (!rmask) return;
+  float ck[2];
+  bool okk[2];
+  {
+    uint64_t one[2][kEPT], m1[2];
+    bool set1[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      const uint32_t n = ((lmask >> s) & 1u) ? f.aux[s].n : 0u;
 #pragma unroll
-      for (int q = 0; q < kEPT; ++q) {
-        const uint32_t e = static_cast<uint32_t>(threadIdx.x + kFW * q);
-        eb1[s][q] = e < n ? f.ent[s].pbits[e] : 0u;
-        ew1[s][q] = eb1[s][q] != 0u ? 1u : 0u;
-      }
+      for (int q = 0; q < kEPT; ++q) one[s][q] = eb[s][q] != 0u ? 1u : 0u;
     }
-    const uint64_t thr[2] = {kk, kk};
-    uint64_t m1[2];
-    bool set1[2];
-    select_entries<false>(f, lmask, thr, eb1, ew1, false, ck, m1, okk, set1);
+    const uint64_t k2[2] = {kk, kk};
+    select_entries<false>(f, rmask, k2, eb, one, false, ck, m1, okk, set1);
   }
-  uint32_t flags[2];
-  float cut[2];
-  uint64_t mass[2] = {0u, 0u};
-  uint32_t emask = 0, slow = 0;
+  uint32_t kmask = 0;  // rows whose k largest are entries
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    flags[s] = fl[s];
-    cut[s] = cp[s];
-    if (fl[s] & kRowEmpty) continue;
-    const bool joint = (fl[s] & kRowFiltered) != 0;
-    if (joint && (fl[s] & kRowList)) {
+    if (((rmask >> s) & 1u) && okk[s] && ck[s] > bmax[s]) kmask |= 1u << s;
+  }
+  uint64_t mass[2] = {0u, 0u};
+  if (kmask) entries_mass2(f, kmask, ck, eb, ew, mass);
+  // rows that still need a top-p select: those whose mass at and above ck
+  // reaches thr, and those whose ck is not known to be the row's
+  uint32_t pmask = 0;
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    if (((mask >> s) & 1u) && !(((kmask >> s) & 1u) && mass[s] < thr[s])) pmask |= 1u << s;
+  }
+  if (pmask) resolve_rows<DT, false>(p, f, rows, K, pmask, thr, eb, ew, false);
+  uint32_t fl[2];
+  float cp[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    fl[s] = f.aux[s].flags;
+    cp[s] = ((pmask >> s) & 1u) ? f.aux[s].cut : 0.0f;
+  }
+  uint32_t store = 0, emask = 0, whole = 0;
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    if (!((rmask >> s) & 1u)) continue;
+    if ((kmask >> s) & 1u) {
+      if (!((pmask >> s) & 1u)) store |= 1u << s;  // else cp >= ck: as resolved
+    } else if (((pmask >> s) & 1u) && (fl[s] & kRowList)) {
       if (okk[s] && ck[s] > cp[s]) {
-        cut[s] = ck[s];
+        store |= 1u << s;
         emask |= 1u << s;
-      } else {
-        mass[s] = f.aux[s].mass_fx;
       }
-    } else if (!joint && okk[s] && ck[s] > bmax[s]) {
-      flags[s] = kRowFiltered | kRowList;
-      cut[s] = ck[s];
-      emask |= 1u << s;
     } else {
-      slow |= 1u << s;
+      whole |= 1u << s;
     }
   }
   if (emask) {
     uint64_t em[2];
-    entries_mass2(f, emask, cut, em);
+    entries_mass2(f, emask, ck, eb, ew, em);
     if (emask & 1u) mass[0] = em[0];
     if (emask & 2u) mass[1] = em[1];
   }
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    if (!((slow >> s) & 1u)) continue;
-    // the k-th largest of the whole row by passes over it
-    flags[s] = kRowFiltered | kRowSlow;
-    float c;
-    uint64_t cnt;
-    select_row<DT, true>(p, f, rows[s], K[s], kk, &c, &cnt);
-    cut[s] = c > cp[s] ? c : cp[s];
-    if (collect_support<DT>(p, f, s, rows[s], K[s], cut[s])) {
-      flags[s] |= kRowList;
-      uint64_t em[2];
-      entries_mass2(f, 1u << s, cut, em);
-      mass[s] = em[s];
-    } else {
-      mass[s] = row_mass<DT>(p, f, rows[s], K[s], cut[s]);
-    }
-  }
+  __syncthreads();  // every read of the rows' state above precedes the stores
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      if (fl[s] & kRowEmpty) continue;
-      RowAux& a = f.aux[s];
-      a.flags = flags[s];
-      a.cut = cut[s];
-      a.mass_fx = mass[s];
-      a.mass_f = mass_to_f32(mass[s]);
+      if ((store >> s) & 1u) store_row(f.aux[s], kRowFiltered | kRowList, ck[s], mass[s]);
     }
+  }
+#pragma unroll 1
+  for (int s = 0; s < 2; ++s) {
+    if (!((whole >> s) & 1u)) continue;
+    // the k-th largest of the whole row by passes over it
+    const int row = s == 0 ? rows[0] : rows[1];
+    const RowK Ks = s == 0 ? K[0] : K[1];
+    const float lower = s == 0 ? cp[0] : cp[1];
+    float c;
+    uint64_t m;
+    select_row<DT, true>(p, f, s, row, Ks, kk, 0.0f, &c, &m);
+    c = c > lower ? c : lower;
+    m = row_mass<DT>(p, f, row, Ks, c);
+    if (threadIdx.x == 0) store_row(f.aux[s], kRowFiltered, c, m);
   }
   __syncthreads();
 }
@@ -2033,29 +2394,39 @@ __device__ __forceinline__ int64_t draw_list(const Params& p, FS& f, const uint6
   return f.token;
 }
 
-// Dense-mode draw over the whole vocabulary with weights wfn(i) (slow path).
-template <int DT, typename WFn, class FS>
-__device__ __forceinline__ int64_t draw_dense(const Params& p, FS& f, const char* rowp, const uint32_t* bm, float u, WFn wfn) {
+// Dense-mode draw over the whole vocabulary with weights wfn(x0, x1), zero
+// for every x0 below lo (kPair: x1 is row1's logit at the same index): each
+// chunk's mass by one wave, then the chunk holding the target by positions.
+template <int DT, bool kPair, typename WFn, class FS>
+__device__ __forceinline__ int64_t draw_dense(const Params& p, FS& f, int row0, int row1, float lo, float u, WFn wfn) {
   const int t = threadIdx.x;
-  for (int j = t; j < p.nch; j += kFW) f.csum[j] = 0;
+  const char* r0 = row_ptr(p, row0);
+  const char* r1 = kPair ? row_ptr(p, row1) : nullptr;
+  const uint32_t* bm = row_bitmap(p, row0);
+  uint32_t* q = wave_queue(f);
   if (t == 0) f.token = 0;
-  __syncthreads();
-  row_pass<DT>(p, rowp, bm, 0, p.vocab, [&](int64_t i, float x) {
-    const uint64_t w = wfn(i, x);
-    if (w) __hip_atomic_fetch_add(&f.csum[i >> 11], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  each_chunk<DT, kPair, FS>(p, r0, r1, [&](int j, const ChunkData<DT>& c, const ChunkData<DT>& c1) {
+    constexpr int kBeside = kPair ? kPairX : kAlone;
+    uint64_t own = 0;
+    chunk_pass<DT, kBeside>(p, c, c1, bm, j, lo, __builtin_inff(), q, [&](const Batch<kBeside>& b) {
+#pragma unroll
+      for (int k = 0; k < b.kN; ++k) own += b.valid[k] ? wfn(b.x[k], __uint_as_float(b.beside[k])) : 0u;
+    });
+    own = wave_sum_u64(own);
+    if ((t & (kWave - 1)) == 0) f.csum[j] = own;
   });
   __syncthreads();
   pick_chunk(p, f, u);
   const uint32_t js = f.pick;
   if (js == kNone) return 0;
   const int64_t c0 = static_cast<int64_t>(js) * kChunk;
-  uint64_t w[kPosPT];
+  uint64_t wt[kPosPT];
 #pragma unroll
-  for (int q = 0; q < kPosPT; ++q) {
-    const int64_t i = c0 + kPosPT * t + q;
-    w[q] = i < p.vocab ? wfn(i, load_x<DT>(p, rowp, bm, i)) : 0;
+  for (int r = 0; r < kPosPT; ++r) {
+    const int64_t i = c0 + kPosPT * t + r;
+    wt[r] = i < p.vocab ? wfn(load_x<DT>(p, r0, bm, i), kPair ? load_x<DT>(p, r1, bm, i) : 0.0f) : 0u;
   }
-  pick_in_chunk(f, c0, w, f.pick_rem);
+  pick_in_chunk(f, c0, wt, f.pick_rem);
   return f.token;
 }
 
@@ -2072,6 +2443,11 @@ __device__ __forceinline__ float q_at(const Params& p, const FS& f, const RowK& 
   return filtered_of(a, pval(K1, load_x<DT>(p, row_ptr(p, row1), row_bitmap(p, row1), x)));
 }
 
+// A logit every element of the row's support lies at or above.
+__device__ __forceinline__ float support_floor(const RowAux& a, const RowK& K) {
+  return (a.flags & kRowFiltered) ? x_floor(K, a.cut) : -__builtin_inff();
+}
+
 // Draw from slot 0's filtered distribution P (bonus / sample).
 template <int DT, class FS>
 __device__ __forceinline__ int64_t draw_target(const Params& p, FS& f, int row0, const RowK& K0, float u) {
@@ -2086,8 +2462,8 @@ __device__ __forceinline__ int64_t draw_target(const Params& p, FS& f, int row0,
     }
     return draw_list(p, f, wl, u, !(a.flags & kRowRefilled));
   }
-  return draw_dense<DT>(p, f, row_ptr(p, row0), row_bitmap(p, row0), u,
-                        [&](int64_t, float x) { return fx46(filtered_of(a, pval(K0, x))); });
+  return draw_dense<DT, false>(p, f, row0, row0, support_floor(a, K0), u,
+                               [&](float x, float) { return fx46(filtered_of(a, pval(K0, x))); });
 }
 
 // Residual draw at a rejected position: normalize(max(P - Q, 0)), falling
@@ -2156,31 +2532,37 @@ __device__ __forceinline__ int64_t draw_residual(const Params& p, FS& f, int row
     return draw_list(p, f, wl, u, !(a.flags & kRowRefilled));
   }
   // dense target support: passes over both rows
-  const char* r0 = row_ptr(p, row0);
-  const char* r1 = row_ptr(p, row1);
-  const uint32_t* bm0 = row_bitmap(p, row0);
-  const uint32_t* bm1 = row_bitmap(p, row1);
   const RowAux a1 = f.aux[1];
-  auto dval = [&](int64_t i, float x0) -> float {
-    const float P = filtered_of(a, pval(K0, x0));
-    if (!(P > 0.0f)) return 0.0f;
-    const float Q = (a1.flags & kRowEmpty) ? 0.0f : filtered_of(a1, pval(K1, load_x<DT>(p, r1, bm1, i)));
-    const float d = P - Q;
-    return d > 0.0f ? d : 0.0f;
+  auto pair = [&](float x0, float x1, float* P) -> float {
+    *P = filtered_of(a, pval(K0, x0));
+    const float Q = (a1.flags & kRowEmpty) ? 0.0f : filtered_of(a1, pval(K1, x1));
+    const float d = *P - Q;
+    return *P > 0.0f && d > 0.0f ? d : 0.0f;
   };
+  const float lo = support_floor(a, K0);
+  const char* r1 = row_ptr(p, row1);
+  const uint32_t* bm = row_bitmap(p, row0);
+  uint32_t* qu = wave_queue(f);
   uint64_t dsum = 0, psum = 0;
-  row_pass<DT>(p, r0, bm0, 0, p.vocab, [&](int64_t i, float x0) {
-    dsum += fx46(dval(i, x0));
-    psum += fx46(filtered_of(a, pval(K0, x0)));
+  each_chunk<DT, true, FS>(p, row_ptr(p, row0), r1, [&](int j, const ChunkData<DT>& c, const ChunkData<DT>& c1) {
+    chunk_pass<DT, kPairX>(p, c, c1, bm, j, lo, __builtin_inff(), qu, [&](const Batch<kPairX>& b) {
+#pragma unroll
+      for (int k = 0; k < b.kN; ++k) {
+        float P;
+        const float d = pair(b.x[k], __uint_as_float(b.beside[k]), &P);
+        dsum += b.valid[k] ? fx46(d) : 0u;
+        psum += b.valid[k] ? fx46(P) : 0u;
+      }
+    });
   });
-  const uint64_t dtot = block_sum(dsum, f.red[0]);
-  const uint64_t ptot = block_sum(psum, f.red[1]);
+  uint64_t dtot, ptot;
+  block_sum2(dsum, psum, f.red[1], &dtot, &ptot);
   const bool use_d = dtot > 0;
   const float den = use_d ? mass_to_f32(dtot) : (ptot > 0 ? mass_to_f32(ptot) : 1.0f);
-  __syncthreads();
-  return draw_dense<DT>(p, f, r0, bm0, u, [&](int64_t i, float x0) -> uint64_t {
-    const float w = use_d ? dval(i, x0) : filtered_of(a, pval(K0, x0));
-    return fx46(w / den);
+  return draw_dense<DT, true>(p, f, row0, row1, lo, u, [&](float x0, float x1) -> uint64_t {
+    float P;
+    const float d = pair(x0, x1, &P);
+    return fx46((use_d ? d : P) / den);
   });
 }
 
@@ -2269,12 +2651,15 @@ __device__ __forceinline__ void fin_unit(const Params& p, FS& f) {
   }
   uint32_t eb[2][kEPT];
   uint64_t ew[2][kEPT];
-  place_entries(p, f, nr, sl, mask, eb, ew);
+  place_entries(p, f, nr, sl, kTopK ? 0u : mask, eb, ew);
   __syncthreads();
   RowK K[2];
   for (int s = 0; s < 2; ++s) K[s] = RowK{f.aux[s < nr ? s : 0].mcmax, f.aux[s < nr ? s : 0].s, p.cd};
-  resolve_rows<DT>(p, f, nr, rows, K, mask, thr, eb, ew);
-  if constexpr (kTopK) apply_top_k<DT>(p, f, nr, rows, K);
+  if constexpr (kTopK) {
+    resolve_top_k<DT>(p, f, nr, rows, K, mask, thr, eb, ew);
+  } else {
+    resolve_rows<DT, true>(p, f, rows, K, mask, thr, eb, ew, true);
+  }
 
   if (p.mode == kModeSpec) {
     const int k = p.k;
@@ -2289,7 +2674,7 @@ __device__ __forceinline__ void fin_unit(const Params& p, FS& f) {
       const float Q = a1.has_tok ? filtered_of(a1, a1.ptok) : 0.0f;
       acc = accept_draw(u_acc, P, Q);
       // the draft's support by vocabulary index, for the residual's Q lookups
-      if (!acc && (a1.flags & kRowList)) hash_support(f);
+      if (!acc && (a0.flags & kRowList) && (a1.flags & kRowList)) hash_support(f);
       token = acc ? xdraft : draw_residual<DT>(p, f, rows[0], rows[1], K[0], K[1], u_draw);
     }
     // publish, then the last of the batch element's k+1 units completes the
