@@ -9,28 +9,33 @@
 //
 // Both operands are K-contiguous (hidden [M, H] row-major, weight [V, H] as
 // nn.Linear stores it), so each MFMA operand fragment is one 16-byte load.
-// One 512-lane workgroup computes a 320-row x 192-column tile with
-// v_mfma_f32_16x16x32_bf16: eight waves (two per SIMD) form a 4 (rows) x 2
-// (columns) grid, each wave 5 x 6 tiles of 16 x 16 (120 accumulator
-// registers), so a k-step reads 11 operand fragments from LDS for 30 MFMAs
-// (a 5 x 3 tile per wave reads 8 for 15: about 30 % more LDS traffic per
-// flop, above the LDS read rate at the MFMA peak). Both operands are
-// staged through LDS in k-blocks of 64 (16-byte chunks XOR-swizzled by row):
-// both by direct global-to-LDS loads (global_load_lds_dwordx4), the weight
-// two blocks ahead into a ring of three buffers (non-temporal: read once), so
-// two blocks of HBM reads are in flight while one is multiplied and no
-// registers hold them, the hidden rows (L2-resident, re-read by every column
-// block) one block ahead into two buffers. Each block ends with an explicit
-// wait that leaves the newest block's weight loads in flight and a bare
-// s_barrier (a workgroup fence would wait for them too). The loads bound the
-// kernel (without the MFMAs it takes about 85 % of its time); the hidden rows
-// take 62.5 % of the LDS, which holds the weight ring at three blocks (about
-// 48 KB in flight per CU), and every wave issues a share of both operands'
-// loads. The epilogue reduces each
-// row's (value, -index) key over the tile's columns (in-lane over the six
-// column tiles, shuffles over the 16 lanes of a row, LDS over the two column
-// waves) and writes one key per (column block, row); a second kernel reduces
-// a row's keys to its index.
+// Up to 32 rows go to lm_head_rows_kernel (below): a read of the weight. More
+// go to lm_head_kernel<MT>: one 512-lane workgroup computes a 64 MT-row x
+// 192-column tile with v_mfma_f32_16x16x32_bf16, MT = 1..5 by the rows; eight
+// waves (two per SIMD) form a 4 (rows) x 2 (columns) grid, each wave MT x 6
+// tiles of 16 x 16. At MT = 5 a k-step reads 11 operand fragments from LDS for
+// 30 MFMAs (a 5 x 3 tile per wave reads 8 for 15: about 30 % more LDS traffic
+// per flop, above the LDS read rate at the MFMA peak). Both operands are staged
+// through LDS in k-blocks of 64 (16-byte chunks XOR-swizzled by row) by direct
+// global-to-LDS loads (global_load_lds_dwordx4): the weight two or three blocks
+// ahead (non-temporal: read once), so that those HBM reads are in flight while
+// a block is multiplied and no registers hold them, the hidden rows
+// (L2-resident, re-read by every column block) one or two blocks ahead. Each
+// block ends with an explicit wait that leaves the newest loads in flight and a
+// bare s_barrier (a workgroup fence would wait for them too). The loads bound
+// the kernel (without the MFMAs it takes about 85 % of its time at 320 rows):
+// a wave's loads return in order, so waiting for the next hidden block also
+// waits for every weight load issued before it. Splitting the two operands'
+// loads over different waves, with the next half block's fragments read during
+// a half block's MFMAs, measured slower at 320 rows (68 us against 63): the
+// weight loads of three waves take longer than the same loads spread over
+// eight. Rows and time (H 2048, V 49152, with the finish kernel; before: one
+// 320-row tile for any row count): 3: 61 -> 45 us, 64: 61 -> 50, 128: 61 -> 49,
+// 192: 65 -> 53, 256: 65 -> 60, 320: 66 -> 66, 700: 188 -> 147.
+// The epilogue reduces each row's (value, -index) key over the tile's columns
+// (in-lane over the six column tiles, shuffles over the 16 lanes of a row, LDS
+// over the two column waves) and writes one key per (column block, row); a
+// second kernel reduces a row's keys to its index.
 #include <string>
 
 #include "ls_common.hpp"
@@ -44,16 +49,13 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kLmLanes = 512;
 constexpr int kLmWaves = kLmLanes / 64;         // 8: 4 (rows) x 2 (columns)
-constexpr int kLmMT = 5;                       // 16-row tiles per wave
 constexpr int kLmNT = 6;                       // 16-column tiles per wave
-constexpr int kLmRowsPerWave = 16 * kLmMT;     // 80
 constexpr int kLmColsPerWave = 16 * kLmNT;     // 96
-constexpr int kLmBM = 4 * kLmRowsPerWave;      // 320 rows per workgroup
+constexpr int kLmMaxRows = 320;                // rows per workgroup: 64 MT for MT = 3, 4 or 5 16-row tiles per wave
 constexpr int kLmBN = 2 * kLmColsPerWave;      // 192 columns per workgroup
 constexpr int kLmKB = 64;                      // k per LDS block
+constexpr int kXcds = 8;
 constexpr int kLmRowBytes = kLmKB * 2;         // 128 bytes of a row's k-block
-constexpr int kLmARounds = 5;  // 40 x 1 KB per A block over 8 waves
-static_assert(kLmBM * kLmRowBytes == 40 * 1024 && kLmBN * kLmRowBytes == 24 * 1024, "1 KB rounds per block");
 constexpr int kLmBRounds = 3;  // 24 x 1 KB per B block over 8 waves
 
 struct LmParams {
@@ -63,6 +65,7 @@ struct LmParams {
   int64_t ws;
   int64_t M, H, V;
   int nblk;             // column blocks (ceil(V / 192))
+  int mblk;             // row blocks (ceil(M / 320))
   uint64_t* keys;       // [nblk, M] partial keys
   int64_t* out;         // [M]
   void* logits;         // logits epilogue: [M, V] float32 or bf16, row stride los elements
@@ -73,12 +76,8 @@ struct LmParams {
 // the tile's columns (the argmax and verify paths), or the logits themselves.
 enum LmEpilogue : int { kLmKeys = 0, kLmLogitsF32 = 1, kLmLogitsBF16 = 2 };
 
-constexpr int kLmABytes = kLmBM * kLmRowBytes;  // 40 KB
 constexpr int kLmBBytes = kLmBN * kLmRowBytes;  // 24 KB
-static_assert(kLmBM * 2 * 8 <= kLmABytes, "epilogue keys fit an A buffer");
-static_assert(kLmARounds * kLmWaves == 40 && kLmBRounds * kLmWaves == 24, "whole rounds per wave");
-
-
+static_assert(kLmBRounds * kLmWaves * 1024 == kLmBBytes, "whole rounds per wave");
 
 // Direct global-to-LDS load of 16 bytes per lane: lane l's bytes land at LDS
 // address lds + 16 l (lds wave-uniform, passed in M0, which the compiler sets
@@ -100,16 +99,38 @@ __device__ __forceinline__ void dma16_stream(const void* src, uint32_t lds) {
 // Byte offset of 16-byte chunk c of row r in an A block.
 __device__ __forceinline__ int a_off(int r, int c) { return r * kLmRowBytes + ((c ^ (r & 7)) << 4); }
 
-template <int EPI>
+// More than 128 rows; a workgroup takes kBM of them.
+template <int MT, int EPI>
 __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
-  // separate arrays, so that the compiler's wait for a direct load into one
-  // weight buffer does not hold up reads of the others
-  __shared__ __attribute__((aligned(16))) uint8_t a0[kLmABytes], a1[kLmABytes];
-  __shared__ __attribute__((aligned(16))) uint8_t b0[kLmBBytes], b1[kLmBBytes], b2[kLmBBytes];
+  constexpr int kRowsPerWave = 16 * MT;
+  constexpr int kBM = 4 * kRowsPerWave;
+  constexpr int kABytes = kBM * kLmRowBytes;
+  constexpr int kARounds = kABytes / 1024 / kLmWaves;  // 1 KB loads per wave and block
+  // blocks of hidden rows and of weight in LDS: with up to 192 rows there is
+  // room for a third (and up to 128 for a fourth weight block), so that a load
+  // has two block times to arrive instead of one
+  constexpr int kAStages = MT <= 3 ? 3 : 2, kBStages = MT <= 2 ? 4 : 3;
+  constexpr int kALead = kAStages - 1, kBLead = kBStages - 1;  // blocks ahead
+  // this wave's loads newer than block kb + 1's at the end of block kb
+  constexpr int kNewer = (kALead - 1) * (kARounds + kLmBRounds) + (kBLead > kALead ? kLmBRounds : 0);
+  __shared__ __attribute__((aligned(16))) uint8_t abuf[kAStages][kABytes];
+  __shared__ __attribute__((aligned(16))) uint8_t bbuf[kBStages][kLmBBytes];
   const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
   const int wm = wid >> 1, wn = wid & 1;
-  const int nblk = static_cast<int>(blockIdx.x);
-  const int64_t m_base = static_cast<int64_t>(blockIdx.y) * kLmBM;
+  // Workgroups go to the eight XCDs in turn; the row blocks of one column block
+  // follow each other on one XCD, so its weight comes from HBM once and the
+  // other row blocks read it from that XCD's L2. (With the row block slowest
+  // the whole weight was streamed once per row block: 1260 us against 1120 at
+  // M 1280, H 4096, V 128256. Giving each XCD a run of column blocks of one row
+  // block, for its hidden rows to stay in L2, measured 1160.)
+  int m_blk = 0, nblk = static_cast<int>(blockIdx.x);
+  if (p.mblk > 1) {
+    const int xcd = nblk & (kXcds - 1), at = nblk / kXcds;
+    m_blk = at % p.mblk;
+    nblk = at / p.mblk * kXcds + xcd;
+    if (nblk >= p.nblk) return;
+  }
+  const int64_t m_base = static_cast<int64_t>(m_blk) * kBM;
   const int64_t n_base = static_cast<int64_t>(nblk) * kLmBN;
   const int nkb = static_cast<int>(p.H / kLmKB);
 
@@ -121,9 +142,9 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
   // results are never used). Byte offsets from the block's first row.
   const uint32_t lchunk = static_cast<uint32_t>(((lane & 7) ^ ((lane >> 3) & 7)) << 4);
   const char* abase = p.hidden + m_base * p.hs * 2;
-  uint32_t aoff[kLmARounds];
+  uint32_t aoff[kARounds];
 #pragma unroll
-  for (int i = 0; i < kLmARounds; ++i) {
+  for (int i = 0; i < kARounds; ++i) {
     const int r = (i * kLmWaves + wid) * 8 + (lane >> 3);
     const int64_t rr = m_base + r < p.M ? r : p.M - 1 - m_base;
     aoff[i] = static_cast<uint32_t>(rr * p.hs * 2) + lchunk;
@@ -139,7 +160,7 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
   auto dma_a = [&](int kb, uint8_t* dst) {
     const char* base = abase + static_cast<int64_t>(kb) * kLmRowBytes;
 #pragma unroll
-    for (int i = 0; i < kLmARounds; ++i) {
+    for (int i = 0; i < kARounds; ++i) {
       const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst)) + (i * kLmWaves + wid) * 1024;
       dma16(base + aoff[i], __builtin_amdgcn_readfirstlane(lds));
     }
@@ -153,16 +174,16 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
     }
   };
 
-  f32x4 acc[kLmMT][kLmNT];
+  f32x4 acc[MT][kLmNT];
 #pragma unroll
-  for (int mt = 0; mt < kLmMT; ++mt) {
+  for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
     for (int nt = 0; nt < kLmNT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   // fragment rows: this wave's first row / column plus lane & 15 (tiles are a
   // multiple of 16 rows apart, so the swizzle is fixed per lane and the rest
   // is an immediate offset)
-  const int fr_a = (wm * kLmRowsPerWave + (lane & 15)) * kLmRowBytes;
+  const int fr_a = (wm * kRowsPerWave + (lane & 15)) * kLmRowBytes;
   const int fr_b = (wn * kLmColsPerWave + (lane & 15)) * kLmRowBytes;
   // One k-block: 2 k-steps x 5 row tiles. Each tile's fragment (and each
   // k-step's column fragments) is read one tile ahead, before the current
@@ -183,10 +204,10 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
     read_b(0, bcur);
     acur = read_a(0, 0);
 #pragma unroll
-    for (int g = 0; g < 2 * kLmMT; ++g) {
-      const int ks = g / kLmMT, mt = g % kLmMT;
-      if (g + 1 < 2 * kLmMT) {
-        const int ks1 = (g + 1) / kLmMT, mt1 = (g + 1) % kLmMT;
+    for (int g = 0; g < 2 * MT; ++g) {
+      const int ks = g / MT, mt = g % MT;
+      if (g + 1 < 2 * MT) {
+        const int ks1 = (g + 1) / MT, mt1 = (g + 1) % MT;
         if (ks1 != ks) read_b(ks1, bnext);
         anext = read_a(ks1, mt1);
       }
@@ -195,20 +216,19 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
         acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(acur, bcur[nt], acc[mt][nt], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       acur = anext;
-      if (g + 1 == kLmMT) {
+      if (g + 1 == MT) {
 #pragma unroll
         for (int nt = 0; nt < kLmNT; ++nt) bcur[nt] = bnext[nt];
       }
     }
   };
-  // End of block kb: every direct load but the newest weight block's (this
-  // wave's kLmBRounds of them, when issued) has landed in LDS, this lane's
-  // LDS reads are done, then the workgroup meets.
-  static_assert(kLmBRounds == 3, "the wait below leaves three loads in flight");
-  auto block_end = [&](bool newest_in_flight) {
+  // End of block kb: block kb + 1 has landed in LDS (loads return in order;
+  // the kNewer newer ones of this wave may be under way), this lane's LDS reads
+  // are done, then the workgroup meets.
+  auto block_end = [&](bool newer_in_flight) {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    if (newest_in_flight) {
-      __builtin_amdgcn_s_waitcnt(0x0073);  // vmcnt(3) expcnt(7) lgkmcnt(0)
+    if (newer_in_flight) {
+      __builtin_amdgcn_s_waitcnt((kNewer & 15) | ((kNewer >> 4) << 14) | 0x70);  // vmcnt(kNewer) lgkmcnt(0)
     } else {
       __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) expcnt(7) lgkmcnt(0)
     }
@@ -216,26 +236,27 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
   };
 
-
-  // block kb: hidden rows in a[kb & 1], weight rows in b[kb % 3]; unrolled by
-  // six so that every buffer is named statically. Per block, the hidden rows
-  // of kb + 1, then the weight rows of kb + 2, go out before kb is multiplied,
-  // and block_end leaves only the latter in flight.
-  dma_a(0, a0);
-  dma_b(0, b0);
-  if (nkb > 1) dma_b(1, b1);
-  block_end(nkb > 1);
-  uint8_t* const A[2] = {a0, a1};
-  uint8_t* const B[3] = {b0, b1, b2};
-  for (int kb0 = 0; kb0 < nkb; kb0 += 6) {
+  // block kb: hidden rows in abuf[kb % kAStages], weight rows in bbuf[kb %
+  // kBStages]; unrolled so that every buffer is named statically. Per block,
+  // the hidden rows of kb + kALead, then the weight rows of kb + kBLead, go out
+  // before kb is multiplied, into buffers last read a barrier ago.
 #pragma unroll
-    for (int u = 0; u < 6; ++u) {
+  for (int i = 0; i < kBLead; ++i) {
+    if (i < kALead && i < nkb) dma_a(i, abuf[i]);
+    if (i < nkb) dma_b(i, bbuf[i]);
+  }
+  block_end(false);
+  constexpr int kUnroll = MT <= 2 ? 12 : (MT == 3 ? 3 : 6);  // whole turns of both rings
+  static_assert(kUnroll % kAStages == 0 && kUnroll % kBStages == 0, "static buffers");
+  for (int kb0 = 0; kb0 < nkb; kb0 += kUnroll) {
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
       const int kb = kb0 + u;
       if (kb < nkb) {
-        if (kb + 1 < nkb) dma_a(kb + 1, A[(u + 1) & 1]);
-        const bool ahead = kb + 2 < nkb;
-        if (ahead) dma_b(kb + 2, B[(u + 2) % 3]);
-        compute(A[u & 1], B[u % 3]);
+        if (kb + kALead < nkb) dma_a(kb + kALead, abuf[(u + kALead) % kAStages]);
+        const bool ahead = kb + kBLead < nkb;
+        if (ahead) dma_b(kb + kBLead, bbuf[(u + kBLead) % kBStages]);
+        compute(abuf[u % kAStages], bbuf[u % kBStages]);
         block_end(ahead);
       }
     }
@@ -245,10 +266,10 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
     // logits: accumulator i of tile (mt, nt) is row (lane / 16) * 4 + i, column
     // lane % 16 of the tile; 16 lanes store 16 consecutive columns of a row
 #pragma unroll
-    for (int mt = 0; mt < kLmMT; ++mt) {
+    for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int64_t m = m_base + wm * kLmRowsPerWave + mt * 16 + (lane >> 4) * 4 + i;
+        const int64_t m = m_base + wm * kRowsPerWave + mt * 16 + (lane >> 4) * 4 + i;
         if (m >= p.M) continue;
 #pragma unroll
         for (int nt = 0; nt < kLmNT; ++nt) {
@@ -264,10 +285,10 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
     }
     return;
   }
-  uint64_t* const keys = reinterpret_cast<uint64_t*>(a0);  // every read of a0 is behind the last barrier
+  uint64_t* const keys = reinterpret_cast<uint64_t*>(abuf);  // every read of it is behind the last barrier
   // epilogue: row keys over this wave's 96 columns, then over the 2 column waves
 #pragma unroll
-  for (int mt = 0; mt < kLmMT; ++mt) {
+  for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       uint64_t best = 0;
@@ -282,16 +303,222 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
         const uint64_t o = __shfl_xor(best, s);
         best = o > best ? o : best;
       }
-      if ((lane & 15) == 0) keys[(wm * kLmRowsPerWave + mt * 16 + (lane >> 4) * 4 + i) * 2 + wn] = best;
+      if ((lane & 15) == 0) keys[(wm * kRowsPerWave + mt * 16 + (lane >> 4) * 4 + i) * 2 + wn] = best;
     }
   }
   __syncthreads();
-  for (int r = t; r < kLmBM; r += kLmLanes) {
+  for (int r = t; r < kBM; r += kLmLanes) {
     const int64_t m = m_base + r;
     if (m < p.M) {
       const uint64_t k0 = keys[r * 2], k1 = keys[r * 2 + 1];
       const uint64_t best = k1 > k0 ? k1 : k0;
       p.keys[static_cast<int64_t>(nblk) * p.M + m] = best;
+    }
+  }
+}
+
+// Up to 32 rows: the weight straight into registers.
+//
+// With few rows the head is a read of the weight (2 V H bytes for 2 M V H
+// flops). Here each of twelve waves owns 16 of the 192 columns; its weight
+// fragments are its own, so they need no LDS: a lane loads them four k-blocks
+// of 64 ahead (8 loads, 32 registers; 96 KB in flight per CU; eight ahead
+// measured the same), in order and without waiting for anything else. The
+// hidden rows, shared by the waves, go through two LDS buffers of four
+// k-blocks, one barrier per buffer. H 2048, V 49152, M = 3: 45 us with the
+// finish kernel against 48.5 for lm_head_kernel<1>, M = 32: 45 against 46; past
+// 32 rows the reads of the hidden rows by every wave cost more than the shared
+// tile's (M = 64: 52 against 50). A read of the same bytes in the same pattern,
+// and nothing else, takes 34.5 us.
+constexpr int kDppRowRor8 = 0x128;
+constexpr int kLrLanes = 768;
+constexpr int kLrWaves = kLrLanes / 64;  // one per 16 columns
+constexpr int kLrAhead = 4;              // k-blocks of weight in flight per wave
+static_assert(kLrWaves * 16 == kLmBN, "the same column blocks as lm_head_kernel (their keys share a layout)");
+
+template <int MT, int EPI>
+__global__ __launch_bounds__(kLrLanes) void lm_head_rows_kernel(const LmParams p) {
+  constexpr int kRows = 16 * MT;
+  constexpr int kSteps = 4;                      // k-blocks per LDS buffer
+  constexpr int kStepBytes = kRows * kLmRowBytes;
+  constexpr int kDeep = kLrAhead / kSteps;       // buffers of hidden rows on their way in registers
+  constexpr int kChunks = kSteps * kStepBytes / 16;
+  constexpr int kRounds = (kChunks + kLrLanes - 1) / kLrLanes;
+  __shared__ __attribute__((aligned(16))) uint8_t abuf[2][kSteps * kStepBytes];
+  __shared__ uint64_t keys[kRows][kLrWaves];
+  const int t = threadIdx.x, lane = t & (kWave - 1);
+  const int w = __builtin_amdgcn_readfirstlane(t / kWave);
+  const int nblk = static_cast<int>(blockIdx.x);
+  const int64_t n_base = static_cast<int64_t>(nblk) * kLmBN;
+  const int nkb = static_cast<int>(p.H / kLmKB);
+  const int64_t col = n_base + w * 16 + (lane & 15);  // of this lane's accumulators
+  // This lane's 16 bytes of weight rows lane & 7 and 8 + (lane & 7) of the
+  // wave's sixteen (clamped: the results of columns past V are not used): one
+  // load takes whole 128-byte lines of eight rows (half lines of sixteen, as the
+  // MFMA has them, read at 4.9-5.3 TB/s instead of 5.8-6.5), lane l the chunk
+  // l / 16 of the first half of its line, or of the second where bit 3 of l is
+  // set.
+  const char* bp[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int64_t n = n_base + w * 16 + h * 8 + (lane & 7);
+    bp[h] = p.weight + (n < p.V ? n : p.V - 1) * p.ws * 2 + (((lane >> 3) & 1) * 4 + (lane >> 4)) * 16;
+  }
+  const char* const none = p.weight;  // what a load past the last k-block reads
+
+  // hidden rows: chunk i = t + 768 r of a buffer is 16 bytes of row (i / 8) mod
+  // kRows of k-block i / (8 kRows), XOR-swizzled by row as in lm_head_kernel
+  const char* ap[kRounds];
+  int astep[kRounds];
+  uint32_t aoff[kRounds];
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int i = t + r * kLrLanes;
+    const int row = (i >> 3) & (kRows - 1), ch = i & 7;
+    astep[r] = i / (8 * kRows);
+    aoff[r] = static_cast<uint32_t>(astep[r] * kStepBytes + a_off(row, ch));
+    ap[r] = p.hidden + (row < p.M ? row : p.M - 1) * p.hs * 2 + ch * 16;
+  }
+  u32x4 areg[kDeep][kRounds];
+  auto load_a = [&](int kb0, u32x4 (&d)[kRounds]) {  // the buffer of k-blocks kb0 .. (past the last: the last again, not used)
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      const int kb = kb0 + astep[r] < nkb ? kb0 + astep[r] : nkb - 1;
+      d[r] = *reinterpret_cast<const u32x4*>(ap[r] + static_cast<int64_t>(kb) * kLmRowBytes);
+    }
+  };
+  auto store_a = [&](uint8_t* buf, const u32x4 (&d)[kRounds]) {
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      if (kChunks % kLrLanes == 0 || t + r * kLrLanes < kChunks) *reinterpret_cast<u32x4*>(buf + aoff[r]) = d[r];
+    }
+  };
+  auto meet = [&]() {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0); the weight loads stay in flight
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  };
+  u32x4 b[kLrAhead][2];
+  auto load_b = [&](int kb, u32x4 (&d)[2]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const char* src = kb < nkb ? bp[h] + static_cast<int64_t>(kb) * kLmRowBytes : none;
+      d[h] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src));
+    }
+  };
+  // Fragments of a k-block's two halves: the first takes rows 0..7 from the
+  // lanes below 8 of each sixteen and rows 8..15 from those lanes of the other
+  // load (rotated by eight), the second the other way round.
+  auto fragments = [&](const u32x4 (&d)[2], bf16x8 (&f)[2]) {
+    u32x4 f0, f1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f0[i] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(d[0][i]), static_cast<int>(d[1][i]),
+                                                                kDppRowRor8, 0xf, 0xc, false));
+      f1[i] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(d[1][i]), static_cast<int>(d[0][i]),
+                                                                kDppRowRor8, 0xf, 0x3, false));
+    }
+    f[0] = __builtin_bit_cast(bf16x8, f0);
+    f[1] = __builtin_bit_cast(bf16x8, f1);
+  };
+  f32x4 acc[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int fr = (lane & 15) * kLmRowBytes;
+  auto multiply = [&](const uint8_t* step, const u32x4 (&d)[2]) {
+    bf16x8 b2[2];
+    fragments(d, b2);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const int sw = ((ks * 4 + (lane >> 4)) ^ (lane & 7)) << 4;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const bf16x8 a = __builtin_bit_cast(
+            bf16x8, *reinterpret_cast<const u32x4*>(step + fr + sw + mt * 16 * kLmRowBytes));
+        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b2[ks], acc[mt], 0, 0, 0);
+      }
+    }
+  };
+
+  // Loads return in order, so hidden rows asked for after a k-block's weight
+  // arrive after it: they go out as far ahead as the weight does (buffer q of
+  // the next group's beside k-block q * kSteps of its weight), or waiting for
+  // them would wait for all the weight under way.
+  u32x4 first[kRounds];
+  load_a(0, first);
+#pragma unroll
+  for (int u = 0; u < kLrAhead; ++u) {
+    load_b(u, b[u]);
+    if (u % kSteps == kSteps - 1) load_a(u + 1, areg[u / kSteps]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  store_a(abuf[0], first);
+  meet();
+  int cur = 0;  // buffer of the k-blocks being multiplied
+  int kb0 = 0;
+  // whole groups of kLrAhead k-blocks with more to come: no branch inside, so
+  // that the compiler's wait for one group's weight leaves the next in flight
+  for (; kb0 + kLrAhead < nkb; kb0 += kLrAhead) {
+#pragma unroll
+    for (int u = 0; u < kLrAhead; ++u) {
+      multiply(abuf[cur] + (u % kSteps) * kStepBytes, b[u]);
+      __builtin_amdgcn_sched_barrier(0);
+      load_b(kb0 + u + kLrAhead, b[u]);
+      if (u % kSteps == kSteps - 1) {
+        store_a(abuf[cur ^ 1], areg[u / kSteps]);
+        load_a(kb0 + u + kLrAhead + 1, areg[u / kSteps]);
+        meet();
+        cur ^= 1;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // the last group (1 .. kLrAhead k-blocks)
+#pragma unroll
+  for (int u = 0; u < kLrAhead; ++u) {
+    if (kb0 + u < nkb) {
+      multiply(abuf[cur] + (u % kSteps) * kStepBytes, b[u]);
+      if (u % kSteps == kSteps - 1 && kb0 + u + 1 < nkb) {
+        store_a(abuf[cur ^ 1], areg[u / kSteps]);
+        meet();
+        cur ^= 1;
+      }
+    }
+  }
+
+  // accumulator i of row tile mt is row mt * 16 + (lane / 16) * 4 + i
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = mt * 16 + (lane >> 4) * 4 + i;
+      if constexpr (EPI == kLmKeys) {
+        uint64_t best = col < p.V ? argmax_key(acc[mt][i], static_cast<uint32_t>(col)) : 0ull;
+#pragma unroll
+        for (int sft = 1; sft < 16; sft <<= 1) {
+          const uint64_t o = __shfl_xor(best, sft);
+          best = o > best ? o : best;
+        }
+        if ((lane & 15) == 0) keys[m][w] = best;
+      } else {
+        if (m < p.M && col < p.V) {
+          if constexpr (EPI == kLmLogitsF32) {
+            static_cast<float*>(p.logits)[m * p.los + col] = acc[mt][i];
+          } else {
+            static_cast<__bf16*>(p.logits)[m * p.los + col] = static_cast<__bf16>(acc[mt][i]);
+          }
+        }
+      }
+    }
+  }
+  if constexpr (EPI == kLmKeys) {
+    __syncthreads();
+    if (t < kRows && t < p.M) {
+      uint64_t best = keys[t][0];
+#pragma unroll
+      for (int i = 1; i < kLrWaves; ++i) best = keys[t][i] > best ? keys[t][i] : best;
+      p.keys[static_cast<int64_t>(nblk) * p.M + t] = best;
     }
   }
 }
@@ -371,6 +598,36 @@ uint64_t ls_lm_head_argmax_workspace(int64_t rows, int64_t vocab) {
 
 namespace {
 
+// The kernel of a head call: a rule on the rows alone, so that every entry
+// point forms a row's logits by the same products in the same order.
+template <int EPI>
+void launch_head(const LmParams& p, hipStream_t st) {
+  if (p.M <= 32) {
+    const dim3 grid(static_cast<unsigned>(p.nblk));
+    if (p.M <= 16) {
+      hipLaunchKernelGGL((lm_head_rows_kernel<1, EPI>), grid, dim3(kLrLanes), 0, st, p);
+    } else {
+      hipLaunchKernelGGL((lm_head_rows_kernel<2, EPI>), grid, dim3(kLrLanes), 0, st, p);
+    }
+    return;
+  }
+  // column blocks in groups of kXcds, each with its row blocks (see the kernel)
+  const int cols = p.mblk > 1 ? (p.nblk + kXcds - 1) / kXcds * kXcds : p.nblk;
+  const dim3 grid(static_cast<unsigned>(cols) * static_cast<unsigned>(p.mblk));
+  const int64_t rows = (p.M + p.mblk - 1) / p.mblk;  // per row block
+  if (rows <= 64) {
+    hipLaunchKernelGGL((lm_head_kernel<1, EPI>), grid, dim3(kLmLanes), 0, st, p);
+  } else if (rows <= 128) {
+    hipLaunchKernelGGL((lm_head_kernel<2, EPI>), grid, dim3(kLmLanes), 0, st, p);
+  } else if (rows <= 192) {
+    hipLaunchKernelGGL((lm_head_kernel<3, EPI>), grid, dim3(kLmLanes), 0, st, p);
+  } else if (rows <= 256) {
+    hipLaunchKernelGGL((lm_head_kernel<4, EPI>), grid, dim3(kLmLanes), 0, st, p);
+  } else {
+    hipLaunchKernelGGL((lm_head_kernel<5, EPI>), grid, dim3(kLmLanes), 0, st, p);
+  }
+}
+
 // Checks shared by the head's entry points; fills p and launches the head
 // kernel (the caller launches the finish kernel it needs).
 int lm_head_launch(const char* what, const void* hidden, int64_t hidden_stride, const void* weight,
@@ -388,7 +645,7 @@ int lm_head_launch(const char* what, const void* hidden, int64_t hidden_stride, 
       hidden_stride < hidden_size || weight_stride < hidden_size)
     return fail(LS_ERR_VALUE, w + ": rows must be 16-byte aligned with strides >= hidden_size");
   const int64_t nblk = (vocab + kLmBN - 1) / kLmBN;
-  const int64_t mblk = (rows + kLmBM - 1) / kLmBM;
+  const int64_t mblk = (rows + kLmMaxRows - 1) / kLmMaxRows;
   if (mblk > 65535) return fail(LS_ERR_VALUE, w + ": too many rows");
   if (epi == kLmKeys && (workspace == nullptr || ws_bytes < ls_lm_head_argmax_workspace(rows, vocab)))
     return fail(LS_ERR_VALUE, w + ": workspace too small");
@@ -404,16 +661,16 @@ int lm_head_launch(const char* what, const void* hidden, int64_t hidden_stride, 
   p.H = hidden_size;
   p.V = vocab;
   p.nblk = static_cast<int>(nblk);
+  p.mblk = static_cast<int>(mblk);
   p.keys = static_cast<uint64_t*>(workspace);
   p.logits = logits;
   p.los = logits_stride;
-  const dim3 grid(static_cast<unsigned>(nblk), static_cast<unsigned>(mblk));
   if (epi == kLmLogitsF32) {
-    hipLaunchKernelGGL(lm_head_kernel<kLmLogitsF32>, grid, dim3(kLmLanes), 0, st, p);
+    launch_head<kLmLogitsF32>(p, st);
   } else if (epi == kLmLogitsBF16) {
-    hipLaunchKernelGGL(lm_head_kernel<kLmLogitsBF16>, grid, dim3(kLmLanes), 0, st, p);
+    launch_head<kLmLogitsBF16>(p, st);
   } else {
-    hipLaunchKernelGGL(lm_head_kernel<kLmKeys>, grid, dim3(kLmLanes), 0, st, p);
+    launch_head<kLmKeys>(p, st);
   }
   return LS_OK;
 }
