@@ -1044,6 +1044,25 @@ struct FinShT {
 
 static_assert(sizeof(FinShT<10>) <= 80 * 1024, "two finaliser workgroups per CU");
 
+// A value every lane holds alike, in scalar registers (the whole-row passes keep
+// a unit's constants over code that needs every vector register).
+__device__ __forceinline__ float uniform(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ uint64_t uniform(uint64_t v) {
+  return pack_u32(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))),
+                  static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32))));
+}
+
+// The thread's index, opaque to the compiler: addresses formed from it are
+// formed again where they are used, not kept in registers from one use to the
+// next over a whole row's select.
+__device__ __forceinline__ int thread_index() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 // Lanes below this one whose bit is set in a wave mask.
 __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32),
@@ -1250,9 +1269,10 @@ __device__ __forceinline__ void row_setup(const Params& p, FS& f, int s, const R
 // were known, placed into the LDS entries when the record's count covers
 // them: entry cstart + k holds (bits of p, vocabulary index). The bits of p
 // and their masses stay in eb / ew (zero for an unused slot); the rows in
-// `hist` add their masses to the bins of the first select round (bits 29..20
+// `hist` add their masses (kCount: their numbers, for the select by counts that
+// comes first with top-k) to the bins of the first select round (bits 29..20
 // of p) and to their coarse sums, which are zero on entry.
-template <class FS>
+template <bool kCount, class FS>
 __device__ __forceinline__ void place_entries(const Params& p, FS& f, int nr, const uint64_t (&sl)[2][kEPT],
                                               uint32_t hist, uint32_t (&eb)[2][kEPT], uint64_t (&ew)[2][kEPT]) {
   const int t = threadIdx.x;
@@ -1284,10 +1304,11 @@ __device__ __forceinline__ void place_entries(const Params& p, FS& f, int nr, co
     if ((hist >> s) & 1u) {
 #pragma unroll
       for (int q = 0; q < kEPT; ++q) {
-        if (ew[s][q] && (eb[s][q] >> 30) == 0u) {
-          __hip_atomic_fetch_add(&f.u.bins[s][eb[s][q] >> (30 - FS::kBits)], ew[s][q], __ATOMIC_RELAXED,
+        const uint64_t w = kCount ? (eb[s][q] != 0u ? 1u : 0u) : ew[s][q];
+        if (w && (eb[s][q] >> 30) == 0u) {
+          __hip_atomic_fetch_add(&f.u.bins[s][eb[s][q] >> (30 - FS::kBits)], w, __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_WORKGROUP);
-          __hip_atomic_fetch_add(&f.coarse[s][eb[s][q] >> (35 - FS::kBits)], ew[s][q], __ATOMIC_RELAXED,
+          __hip_atomic_fetch_add(&f.coarse[s][eb[s][q] >> (35 - FS::kBits)], w, __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_WORKGROUP);
         }
       }
@@ -1319,7 +1340,7 @@ __device__ __forceinline__ void select_entries(FS& f, uint32_t mask, const uint6
                                                const uint32_t (&eb)[2][kEPT], const uint64_t (&ew)[2][kEPT],
                                                bool hist, float (&cut)[2], uint64_t (&mass)[2],
                                                bool (&ok)[2], bool (&set)[2]) {
-  const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
+  const int t = thread_index(), lane = t & (kWave - 1), wid = t / kWave;
   bool live[2] = {(mask & 1u) != 0, (mask & 2u) != 0};
   ok[0] = live[0];
   ok[1] = live[1];
@@ -1530,53 +1551,49 @@ __device__ __forceinline__ void wave_lds_fence() {
 // same index, or the index.
 enum Beside : int { kAlone = 0, kPairX = 1, kIndex = 2 };
 
-// Chunk j of a row as one wave loads it: vector u of lane t (words 4 u .. of
-// its registers) is the chunk's vector 64 u + t (lanes past the chunk's end
-// re-read its last vector). The passes below loop over a chunk's elements a
-// few at a time with a uniform register index, not unrolled over the 32 of a
-// lane: the same time, and a third of the code.
-typedef uint32_t u32x32 __attribute__((ext_vector_type(32)));
+// A piece of a row as one wave loads it: four vectors per lane, vector u of
+// lane t (words 4 u .. of its registers) the piece's vector 64 u + t (lanes past
+// the row's end re-read its last vector); 1024 elements in f32 (two pieces to a
+// chunk), 2048 in 16 bits. bits: with a penalty, the bitmap word of each vector.
+// The passes below loop over a piece's elements a few at a time with a uniform
+// register index, not unrolled: the same time, and a third of the code.
 typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
 template <int DT>
-struct ChunkRegs {
-  using type = u32x16;
-};
-template <>
-struct ChunkRegs<F32> {
-  using type = u32x32;
-};
-template <int DT>
-struct ChunkData {
-  static constexpr int kVecs = kChunk / (kWave * Elem<DT>::kPerVec);
-  typename ChunkRegs<DT>::type d;
+struct Piece {
+  static constexpr int kVecs = 4;
+  static constexpr int kElems = kVecs * kWave * Elem<DT>::kPerVec;
+  static constexpr int kPerChunk = kChunk / kElems;
+  u32x16 d;
+  u32x4 bits;
 };
 
+// Piece q of a row (element q * kElems on).
 template <int DT>
-__device__ __forceinline__ void load_chunk(const Params& p, const char* rowp, int j, ChunkData<DT>& c) {
+__device__ __forceinline__ void load_piece(const Params& p, const char* rowp, const uint32_t* bm, int q, Piece<DT>& c) {
   constexpr int EPV = Elem<DT>::kPerVec;
   const int lane = threadIdx.x & (kWave - 1);
-  const int c0 = j * kChunk;
-  const int nvc = (p.vocab - c0 < kChunk ? p.vocab - c0 : kChunk) / EPV;
-  const u32x4* src = reinterpret_cast<const u32x4*>(rowp) + c0 / EPV;
+  const int v0 = q * Piece<DT>::kElems / EPV, nv = p.vocab / EPV;
+  const u32x4* src = reinterpret_cast<const u32x4*>(rowp);
 #pragma unroll
-  for (int u = 0; u < ChunkData<DT>::kVecs; ++u) {
-    const int v = u * kWave + lane;
-    const u32x4 x = src[v < nvc ? v : nvc - 1];
+  for (int u = 0; u < Piece<DT>::kVecs; ++u) {
+    const int at = v0 + u * kWave + lane, v = at < nv ? at : nv - 1;
+    const u32x4 x = src[v];
 #pragma unroll
     for (int k = 0; k < 4; ++k) c.d[4 * u + k] = x[k];
+    if (bm) c.bits[u] = bm[(v * EPV) >> 5];
   }
 }
 
-// kStep elements of a lane from a chunk's registers, processed: elements
-// kStep * st .. of the lane's 32, whose chunk index is *i0 onwards.
+// kStep elements of a lane from a piece's registers, processed: those from its
+// kStep * st 'th on, whose index in the row is *i0 onwards.
 template <int DT, int kStep>
-__device__ __forceinline__ void chunk_step(const Params& p, const ChunkData<DT>& c, const uint32_t* bm, int j, int st,
+__device__ __forceinline__ void piece_step(const Params& p, const Piece<DT>& c, u32x4 bits, bool pen, int q, int st,
                                            float (&x)[kStep], int* i0) {
   constexpr int EPV = Elem<DT>::kPerVec;
   constexpr int kPerWord = EPV / 4;
   const int lane = threadIdx.x & (kWave - 1);
   const int u = st * kStep / EPV, e0 = st * kStep % EPV;
-  const int i = (u * kWave + lane) * EPV + e0;
+  const int i = q * Piece<DT>::kElems + (u * kWave + lane) * EPV + e0;
 #pragma unroll
   for (int w = 0; w < kStep / kPerWord; ++w) {
     const uint32_t word = c.d[st * (kStep / kPerWord) + w];
@@ -1587,49 +1604,68 @@ __device__ __forceinline__ void chunk_step(const Params& p, const ChunkData<DT>&
       x[2 * w + 1] = bits_to_float<DT>(word >> 16);
     }
   }
-  if (bm) {
-    const int at = j * kChunk + i;
-    const uint32_t pb = at < p.vocab ? bm[at >> 5] >> (at & 31) : 0u;
+  if (pen) {
+    const uint32_t pb = bits[u] >> (i & 31);
 #pragma unroll
     for (int e = 0; e < kStep; ++e) x[e] = (pb >> e) & 1u ? penalise(x[e], p.pen) : x[e];
   }
   *i0 = i;
 }
 
-// What fn of a pass gets at a time: kBatch queued logits per lane, so that
-// the exact p of several are under way together (two waves per SIMD do not
-// hide the latency of one's dependent chain).
-template <int kBeside>
+// What fn of a pass gets at a time: kN queued logits per lane, so that with
+// one workgroup per CU (two waves per SIMD) the exact p of several are under
+// way together; with two workgroups one (their registers are few, and the other
+// waves cover a dependent chain's latency).
+template <int kBeside, class FS>
 struct Batch {
-  static constexpr int kN = kBeside == kAlone ? 4 : 2;
+  static constexpr int kN = FS::kBits > 10 ? (kBeside == kAlone ? 4 : 2) : 1;
   float x[kN];
   uint32_t beside[kN];
   bool valid[kN];
 };
 
-// One wave over loaded chunk j of a row: fn(batch) on the elements whose
+// One wave over loaded piece q of a row: fn(batch) on the elements whose
 // processed logit lies in [lo, hi] (a NaN counts as inside), in no particular
 // order. fn evaluates p exactly (some 32 instructions, in binary64), and a pass
 // wants few of the elements, so each element's test only appends it to the
-// wave's queue in LDS and fn runs on full waves of queued ones. The chunk's
+// wave's queue in LDS and fn runs on full waves of queued ones. The piece's
 // elements are all done on return.
-template <int DT, int kBeside, typename Fn>
-__device__ __forceinline__ void chunk_pass(const Params& p, const ChunkData<DT>& c, const ChunkData<DT>& c1,
-                                           const uint32_t* bm, int j, float lo, float hi, uint32_t* q, Fn fn) {
-  using B = Batch<kBeside>;
+// kWhole: with lo = -inf every element is wanted, and goes to fn without the
+// queue.
+template <int DT, int kBeside, bool kWhole, class FS, typename Fn>
+__device__ __forceinline__ void piece_pass(const Params& p, const Piece<DT>& c, const Piece<DT>& c1, int q, float lo,
+                                           float hi, uint32_t* queue, Fn fn) {
+  using B = Batch<kBeside, FS>;
   constexpr int kWords = kBeside == kAlone ? 1 : 2;
   constexpr int kStep = kBeside == kAlone ? 4 : 2;  // elements between drains
+  constexpr int kSteps = Piece<DT>::kElems / kWave / kStep;
   static_assert((kStep + B::kN) * kWave * kWords <= kQueue, "queue size");
   const int lane = threadIdx.x & (kWave - 1);
-  const int nel = p.vocab - j * kChunk < kChunk ? p.vocab - j * kChunk : kChunk;
+  const bool pen = p.use_pen != 0;
   uint32_t n = 0;  // queued (wave-uniform)
 #pragma unroll 1
-  for (int st = 0; st < 32 / kStep; ++st) {
+  for (int st = 0; st < kSteps; ++st) {
     float x[kStep], x1[kStep];
     int i0;
-    chunk_step<DT, kStep>(p, c, bm, j, st, x, &i0);
-    if constexpr (kBeside == kPairX) chunk_step<DT, kStep>(p, c1, bm, j, st, x1, &i0);
-    const bool in_row = i0 < nel;
+    piece_step<DT, kStep>(p, c, c.bits, pen, q, st, x, &i0);
+    if constexpr (kBeside == kPairX) piece_step<DT, kStep>(p, c1, c.bits, pen, q, st, x1, &i0);
+    const bool in_row = i0 < p.vocab;
+    if constexpr (kWhole) {
+      if (lo == -__builtin_inff()) {
+#pragma unroll
+        for (int e = 0; e < kStep; e += B::kN) {
+          B b;
+#pragma unroll
+          for (int k = 0; k < B::kN; ++k) {
+            b.valid[k] = in_row;
+            b.x[k] = x[e + k];
+            b.beside[k] = kBeside == kPairX ? __float_as_uint(x1[e + k]) : 0u;
+          }
+          fn(b);
+        }
+        continue;
+      }
+    }
 #pragma unroll
     for (int e = 0; e < kStep; ++e) {
       const bool in = in_row && !(x[e] < lo) && !(x[e] > hi);
@@ -1637,15 +1673,15 @@ __device__ __forceinline__ void chunk_pass(const Params& p, const ChunkData<DT>&
       if (in) {
         const uint32_t at = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
                                                       __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), n)) * kWords;
-        q[at] = __float_as_uint(x[e]);
-        if constexpr (kBeside == kPairX) q[at + 1] = __float_as_uint(x1[e]);
-        if constexpr (kBeside == kIndex) q[at + 1] = static_cast<uint32_t>(j * kChunk + i0 + e);
+        queue[at] = __float_as_uint(x[e]);
+        if constexpr (kBeside == kPairX) queue[at + 1] = __float_as_uint(x1[e]);
+        if constexpr (kBeside == kIndex) queue[at + 1] = static_cast<uint32_t>(i0 + e);
       }
       n += static_cast<uint32_t>(__builtin_popcountll(m));
     }
     wave_lds_fence();
     // whole batches; after the last step also the rest
-    const uint32_t most = st == 32 / kStep - 1 ? 0u : B::kN * kWave - 1;
+    const uint32_t most = st == kSteps - 1 ? 0u : B::kN * kWave - 1;
 #pragma unroll 1
     while (n > most) {
       const uint32_t take = n < static_cast<uint32_t>(B::kN * kWave) ? n : static_cast<uint32_t>(B::kN * kWave);
@@ -1656,8 +1692,8 @@ __device__ __forceinline__ void chunk_pass(const Params& p, const ChunkData<DT>&
         const uint32_t i = static_cast<uint32_t>(k * kWave + lane);
         b.valid[k] = i < take;
         const uint32_t at = (n + (b.valid[k] ? i : 0u)) * kWords;
-        b.x[k] = __uint_as_float(q[at]);
-        b.beside[k] = kWords > 1 ? q[at + kWords - 1] : 0u;
+        b.x[k] = __uint_as_float(queue[at]);
+        b.beside[k] = kWords > 1 ? queue[at + kWords - 1] : 0u;
       }
       wave_lds_fence();
       fn(b);
@@ -1665,47 +1701,52 @@ __device__ __forceinline__ void chunk_pass(const Params& p, const ChunkData<DT>&
   }
 }
 
-// The chunk's registers hold their loads' results from here on (otherwise the
-// compiler waits for the loads of the next chunk too wherever this one is read).
+// The piece's registers hold their loads' results from here on (otherwise the
+// compiler waits for the loads of the next piece too wherever this one is read).
 template <int DT>
-__device__ __forceinline__ void chunk_arrived(ChunkData<DT>& c) {
+__device__ __forceinline__ void piece_arrived(Piece<DT>& c) {
   asm volatile("" : "+v"(c.d));
 }
 
-// each(j, chunk, chunk1) over every chunk of a row (kPair: and of a second
-// row), wave w on chunks w, w + kFNW, ... With one workgroup per CU the next
-// chunk's loads are in flight while a chunk is worked on; with two the other
-// waves cover them.
+// each(q, piece, piece1) over every piece of a row (kPair: and of a second
+// row), in chunk order, wave w on chunks w, w + kFNW, ... With one workgroup per
+// CU the next piece's loads are in flight while a piece is worked on; with two
+// the other waves cover them.
 template <int DT, bool kPair, class FS, typename Each>
-__device__ __forceinline__ void each_chunk(const Params& p, const char* row0, const char* row1, Each each) {
+__device__ __forceinline__ void each_piece(const Params& p, const char* row0, const char* row1, const uint32_t* bm,
+                                           Each each) {
   constexpr bool kAhead = FS::kBits > 10;
+  constexpr int kPer = Piece<DT>::kPerChunk;
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
-  ChunkData<DT> c, c1, next, next1;
-  if (w < p.nch) {
-    load_chunk<DT>(p, row0, w, c);
-    if constexpr (kPair) load_chunk<DT>(p, row1, w, c1);
+  const int total = (p.vocab + Piece<DT>::kElems - 1) / Piece<DT>::kElems;  // pieces of the row
+  // the piece after q of this wave's chunks
+  auto after = [&](int q) { return kPer == 1 || q % kPer == kPer - 1 ? q + 1 + (kFNW - 1) * kPer : q + 1; };
+  Piece<DT> c, c1, next, next1;
+  int q = w * kPer;
+  if (q < total) {
+    load_piece<DT>(p, row0, bm, q, c);
+    if constexpr (kPair) load_piece<DT>(p, row1, nullptr, q, c1);
   }
 #pragma unroll 1
-  for (int j = w; j < p.nch; j += kFNW) {
-    if constexpr (!kAhead) {
-      if (j > w) {
-        load_chunk<DT>(p, row0, j, c);
-        if constexpr (kPair) load_chunk<DT>(p, row1, j, c1);
-      }
-    }
-    chunk_arrived<DT>(c);
-    if constexpr (kPair) chunk_arrived<DT>(c1);
+  while (q < total) {
+    const int qn = after(q);
+    piece_arrived<DT>(c);
+    if constexpr (kPair) piece_arrived<DT>(c1);
     if constexpr (kAhead) {
-      if (j + kFNW < p.nch) {
-        load_chunk<DT>(p, row0, j + kFNW, next);
-        if constexpr (kPair) load_chunk<DT>(p, row1, j + kFNW, next1);
+      if (qn < total) {
+        load_piece<DT>(p, row0, bm, qn, next);
+        if constexpr (kPair) load_piece<DT>(p, row1, nullptr, qn, next1);
       }
     }
-    each(j, c, c1);
+    each(q, c, c1);
     if constexpr (kAhead) {
       c = next;
       if constexpr (kPair) c1 = next1;
+    } else if (qn < total) {
+      load_piece<DT>(p, row0, bm, qn, c);
+      if constexpr (kPair) load_piece<DT>(p, row1, nullptr, qn, c1);
     }
+    q = qn;
   }
 }
 
@@ -1714,29 +1755,29 @@ __device__ __forceinline__ uint32_t* wave_queue(FS& f) {
   return f.hash + __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave) * kQueue;
 }
 
-// chunk_pass over every chunk of a row.
+// piece_pass over a whole row.
 template <int DT, class FS, typename Fn>
 __device__ __forceinline__ void row_pass(const Params& p, FS& f, int row, float lo, float hi, Fn fn) {
-  const uint32_t* bm = row_bitmap(p, row);
-  uint32_t* q = wave_queue(f);
-  each_chunk<DT, false, FS>(p, row_ptr(p, row), nullptr, [&](int j, const ChunkData<DT>& c, const ChunkData<DT>&) {
-    chunk_pass<DT, kAlone>(p, c, c, bm, j, lo, hi, q, fn);
-  });
+  uint32_t* queue = wave_queue(f);
+  each_piece<DT, false, FS>(p, row_ptr(p, row), nullptr, row_bitmap(p, row),
+                            [&](int q, const Piece<DT>& c, const Piece<DT>&) {
+                              piece_pass<DT, kAlone, false, FS>(p, c, c, q, lo, hi, queue, fn);
+                            });
 }
 
 // The smallest processed logit of a row (a NaN, whose p is 0, as -inf), per lane.
 template <int DT, class FS>
 __device__ __forceinline__ float lane_row_min(const Params& p, int row) {
   constexpr int kStep = 4;
-  const uint32_t* bm = row_bitmap(p, row);
   float mn = __builtin_inff();
-  each_chunk<DT, false, FS>(p, row_ptr(p, row), nullptr, [&](int j, const ChunkData<DT>& c, const ChunkData<DT>&) {
+  each_piece<DT, false, FS>(p, row_ptr(p, row), nullptr, row_bitmap(p, row),
+                            [&](int q, const Piece<DT>& c, const Piece<DT>&) {
 #pragma unroll 1
-    for (int st = 0; st < 32 / kStep; ++st) {
+    for (int st = 0; st < Piece<DT>::kElems / kWave / kStep; ++st) {
       float x[kStep];
       int i0;
-      chunk_step<DT, kStep>(p, c, bm, j, st, x, &i0);
-      if (j * kChunk + i0 >= p.vocab) continue;
+      piece_step<DT, kStep>(p, c, c.bits, p.use_pen != 0, q, st, x, &i0);
+      if (i0 >= p.vocab) continue;
 #pragma unroll
       for (int e = 0; e < kStep; ++e) mn = x[e] != x[e] ? -__builtin_inff() : (x[e] < mn ? x[e] : mn);
     }
@@ -1747,13 +1788,14 @@ __device__ __forceinline__ float lane_row_min(const Params& p, int row) {
 // Slot s's list entries 0 .. n - 1 selected for `thr` (kCount: by counts).
 template <bool kCount, class FS>
 __device__ __forceinline__ bool select_list(FS& f, int s, uint32_t n, uint64_t thr, float* cut, uint64_t* mass) {
+  const int t = thread_index();
   uint32_t eb[2][kEPT];
   uint64_t ew[2][kEPT];
 #pragma unroll
   for (int s1 = 0; s1 < 2; ++s1) {
 #pragma unroll
     for (int q = 0; q < kEPT; ++q) {
-      const uint32_t e = static_cast<uint32_t>(threadIdx.x + kFW * q);
+      const uint32_t e = static_cast<uint32_t>(t + kFW * q);
       const bool in = s1 == s && e < n;
       eb[s1][q] = in ? f.ent[s].pbits[e] : 0u;
       ew[s1][q] = !in ? 0u : (kCount ? 1u : fx46(__uint_as_float(eb[s1][q])));
@@ -1843,7 +1885,7 @@ template <int DT, class FS>
 __device__ __forceinline__ bool select_window(const Params& p, FS& f, int s, int row, const RowK& K, uint64_t thr,
                                               float v_min, float* cut, uint64_t* mass) {
   constexpr int kStep = 4;
-  const int t = threadIdx.x;
+  const int t = thread_index();
   uint32_t* fb = reinterpret_cast<uint32_t*>(f.u.bins[1]);
   uint64_t* bins = f.u.bins[0];
   const float inf = __builtin_inff();
@@ -1853,17 +1895,17 @@ __device__ __forceinline__ bool select_window(const Params& p, FS& f, int s, int
   if (t == 0) f.gcount[s] = 0;
   __syncthreads();
   {
-    const uint32_t* bm = row_bitmap(p, row);
     const float lo = x_floor(K, v_min);
     // exponents of p in units of 2^-31
     const float c = p.c, nm = 31.0f - K.mcmax - __builtin_amdgcn_logf(K.s);
-    each_chunk<DT, false, FS>(p, row_ptr(p, row), nullptr, [&](int j, const ChunkData<DT>& cd, const ChunkData<DT>&) {
+    each_piece<DT, false, FS>(p, row_ptr(p, row), nullptr, row_bitmap(p, row),
+                              [&](int pq, const Piece<DT>& pc, const Piece<DT>&) {
 #pragma unroll 1
-      for (int st = 0; st < 32 / kStep; ++st) {
+      for (int st = 0; st < Piece<DT>::kElems / kWave / kStep; ++st) {
         float x[kStep];
         int i0;
-        chunk_step<DT, kStep>(p, cd, bm, j, st, x, &i0);
-        const float lo_in = j * kChunk + i0 < p.vocab ? lo : inf;
+        piece_step<DT, kStep>(p, pc, pc.bits, p.use_pen != 0, pq, st, x, &i0);
+        const float lo_in = i0 < p.vocab ? lo : inf;
 #pragma unroll
         for (int e = 0; e < kStep; ++e) {
           if (x[e] >= lo_in) {
@@ -1888,7 +1930,7 @@ __device__ __forceinline__ bool select_window(const Params& p, FS& f, int s, int
   const float v_lo = __uint_as_float((d - 1u + kWinBase) << kWinShift) * 0x1p-31f;
   const float v_hi = __uint_as_float((d + 2u + kWinBase) << kWinShift) * 0x1p-31f;
   uint64_t own = 0;
-  row_pass<DT>(p, f, row, x_floor(K, v_lo), inf, [&](const Batch<kAlone>& b) {
+  row_pass<DT>(p, f, row, x_floor(K, v_lo), inf, [&](const Batch<kAlone, FS>& b) {
     float v[b.kN];
 #pragma unroll
     for (int k = 0; k < b.kN; ++k) {
@@ -1922,7 +1964,7 @@ __device__ __forceinline__ bool select_window(const Params& p, FS& f, int s, int
 template <int DT, bool kCount, class FS>
 __device__ __forceinline__ void select_row(const Params& p, FS& f, int s, int row, const RowK& K, uint64_t thr,
                                            float v_min, float* cut, uint64_t* mass) {
-  const int t = threadIdx.x;
+  const int t = thread_index();
   if constexpr (!kCount) {
     if (select_window<DT>(p, f, s, row, K, thr, v_min, cut, mass)) return;
   }
@@ -1940,7 +1982,7 @@ __device__ __forceinline__ void select_row(const Params& p, FS& f, int s, int ro
     for (int q = 0; q < FS::kPer; ++q) bins[FS::kPer * t + q] = 0;
     if (t == 0) f.gcount[s] = 0;
     __syncthreads();
-    row_pass<DT>(p, f, row, lo, hi, [&](const Batch<kAlone>& b) {
+    row_pass<DT>(p, f, row, lo, hi, [&](const Batch<kAlone, FS>& b) {
 #pragma unroll
       for (int k = 0; k < b.kN; ++k) {
         const uint32_t v = __float_as_uint(pval(K, b.x[k]));
@@ -1970,7 +2012,7 @@ __device__ __forceinline__ void select_row(const Params& p, FS& f, int s, int ro
     // the crossing digit's elements (p from prefix << shift up to the next digit)
     lo = prefix ? x_floor(K, __uint_as_float(prefix << shift)) : -inf;
     hi = x_ceil(K, __uint_as_float((prefix + 1u) << shift));
-    row_pass<DT>(p, f, row, lo, hi, [&](const Batch<kAlone>& b) {
+    row_pass<DT>(p, f, row, lo, hi, [&](const Batch<kAlone, FS>& b) {
 #pragma unroll
       for (int k = 0; k < b.kN; ++k) {
         const uint32_t v = __float_as_uint(pval(K, b.x[k]));
@@ -1994,7 +2036,7 @@ __device__ __forceinline__ void select_row(const Params& p, FS& f, int s, int ro
 // (whose p becomes 0). False when they do not fit. Uses the draft hash's LDS.
 template <int DT, class FS>
 __device__ __forceinline__ bool refill_chunks(const Params& p, FS& f, int s, int row, const RowK& K, float c) {
-  const int t = threadIdx.x, lane = t & (kWave - 1);
+  const int t = thread_index(), lane = t & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(t / kWave);
   const char* rowp = row_ptr(p, row);
   const uint32_t* bm = row_bitmap(p, row);
@@ -2011,22 +2053,29 @@ __device__ __forceinline__ bool refill_chunks(const Params& p, FS& f, int s, int
   int turn = 0;
 #pragma unroll 1
   while (need[0] | need[1]) {
-    const int h = need[0] ? 0 : 1;
-    const int j = h * kWave + __builtin_ctzll(h ? need[1] : need[0]);
-    if (h) need[1] &= need[1] - 1; else need[0] &= need[0] - 1;
+    const int hi = need[0] ? 0 : 1;
+    const int j = hi * kWave + __builtin_ctzll(hi ? need[1] : need[0]);
+    if (hi) need[1] &= need[1] - 1; else need[0] &= need[0] - 1;
     if ((turn++ & (kFNW - 1)) != w) continue;
-    ChunkData<DT> cd;
-    load_chunk<DT>(p, rowp, j, cd);
+    constexpr int kPer = Piece<DT>::kPerChunk;
+    Piece<DT> cd[kPer];
+#pragma unroll
+    for (int h = 0; h < kPer; ++h) load_piece<DT>(p, rowp, bm, j * kPer + h, cd[h]);
     const uint32_t e0 = f.cstart[s][j], e1 = e0 + f.ccount[s][j];
     for (uint32_t e = e0 + lane; e < e1; e += kWave) f.ent[s].pbits[e] = 0u;
-    chunk_pass<DT, kIndex>(p, cd, cd, bm, j, lo, __builtin_inff(), q, [&](const Batch<kIndex>& b) {
-      float v[b.kN];
 #pragma unroll
-      for (int k = 0; k < b.kN; ++k) v[k] = pval(K, b.x[k]);
+    for (int h = 0; h < kPer; ++h) {
+      if ((j * kPer + h) * Piece<DT>::kElems >= p.vocab) break;
+      piece_pass<DT, kIndex, false, FS>(p, cd[h], cd[h], j * kPer + h, lo, __builtin_inff(), q,
+                                 [&](const Batch<kIndex, FS>& b) {
+        float v[b.kN];
 #pragma unroll
-      for (int k = 0; k < b.kN; ++k)
-        list_append<true>(f, s, &f.aux[s].n, b.valid[k] && v[k] >= c, __float_as_uint(v[k]), b.beside[k]);
-    });
+        for (int k = 0; k < b.kN; ++k) v[k] = pval(K, b.x[k]);
+#pragma unroll
+        for (int k = 0; k < b.kN; ++k)
+          list_append<true>(f, s, &f.aux[s].n, b.valid[k] && v[k] >= c, __float_as_uint(v[k]), b.beside[k]);
+      });
+    }
   }
   __syncthreads();
   return f.aux[s].n <= static_cast<uint32_t>(kRowCap);
@@ -2084,7 +2133,8 @@ __device__ __forceinline__ void resolve_rows(const Params& p, FS& f, const int (
       if ((late >> s) & 1u) store_row(f.aux[s], kRowFiltered | kRowList, cut[s], mass[s]);
     }
   }
-  const float g0 = ok[0] ? cut[0] : cutoff_guess(p, thr[0]), g1 = ok[1] ? cut[1] : cutoff_guess(p, thr[1]);
+  const float g0 = uniform(ok[0] ? cut[0] : cutoff_guess(p, thr[0]));
+  const float g1 = uniform(ok[1] ? cut[1] : cutoff_guess(p, thr[1]));
 #pragma unroll 1
   for (int s = 0; s < 2; ++s) {
     if (!((whole >> s) & 1u)) continue;
@@ -2112,14 +2162,16 @@ __device__ __forceinline__ void resolve_rows(const Params& p, FS& f, const int (
 // sum_{p >= c[s]} fx46(p) over the entries of the slots in `mask`, both slots
 // in one block reduction.
 template <class FS>
-__device__ __forceinline__ void entries_mass2(FS& f, uint32_t mask, const float (&c)[2], const uint32_t (&eb)[2][kEPT],
-                                              const uint64_t (&ew)[2][kEPT], uint64_t (&out)[2]) {
+__device__ __forceinline__ void entries_mass2(FS& f, uint32_t mask, const float (&c)[2], uint64_t (&out)[2]) {
   uint64_t own[2] = {0u, 0u};
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     if (!((mask >> s) & 1u)) continue;
-#pragma unroll
-    for (int q = 0; q < kEPT; ++q) own[s] += __uint_as_float(eb[s][q]) >= c[s] ? ew[s][q] : 0u;
+    const uint32_t n = f.aux[s].n;
+    for (uint32_t e = threadIdx.x; e < n; e += kFW) {
+      const float v = __uint_as_float(f.ent[s].pbits[e]);
+      if (v >= c[s]) own[s] += fx46(v);
+    }
   }
   block_sum2(own[0], own[1], f.red[2], &out[0], &out[1]);
   __syncthreads();
@@ -2129,7 +2181,7 @@ __device__ __forceinline__ void entries_mass2(FS& f, uint32_t mask, const float 
 template <int DT, class FS>
 __device__ __forceinline__ uint64_t row_mass(const Params& p, FS& f, int row, const RowK& K, float c) {
   uint64_t own = 0;
-  row_pass<DT>(p, f, row, x_floor(K, c), __builtin_inff(), [&](const Batch<kAlone>& b) {
+  row_pass<DT>(p, f, row, x_floor(K, c), __builtin_inff(), [&](const Batch<kAlone, FS>& b) {
 #pragma unroll
     for (int k = 0; k < b.kN; ++k) {
       const float v = pval(K, b.x[k]);
@@ -2144,7 +2196,8 @@ __device__ __forceinline__ uint64_t row_mass(const Params& p, FS& f, int row, co
 // Cutoffs of the unit's rows with top-k (1 <= p.top_k < V): max(k-th largest
 // p, top-p cutoff) -- the joint rule of distributions.py:72-86, or the k-th
 // largest alone for the rows not in `mask` (top_p = 1) -- with ties kept and
-// one renormalisation over {p >= cutoff}. The k-th largest ck of the entries
+// one renormalisation over {p >= cutoff}. rmask: the rows with any mass, whose
+// entries are counted in the bins already. The k-th largest ck of the entries
 // comes first, by a select by counts over both rows. Above every chunk's
 // non-candidate bound it is the row's, and every element at or above it is an
 // entry, so the top-p cutoff cp is decided there too: the entries' mass at and
@@ -2157,18 +2210,12 @@ __device__ __forceinline__ uint64_t row_mass(const Params& p, FS& f, int row, co
 // elements lie below cp, so its cutoff is max(ck, cp) over the entries; any
 // other row is selected by counts over the whole row.
 template <int DT, class FS>
-__device__ __forceinline__ void resolve_top_k(const Params& p, FS& f, int nr, const int (&rows)[2], const RowK (&K)[2],
-                                              uint32_t mask, const uint64_t (&thr)[2], const uint32_t (&eb)[2][kEPT],
+__device__ __forceinline__ void resolve_top_k(const Params& p, FS& f, const int (&rows)[2], const RowK (&K)[2],
+                                              uint32_t rmask, uint32_t mask, const uint64_t (&thr)[2], const uint32_t (&eb)[2][kEPT],
                                               const uint64_t (&ew)[2][kEPT]) {
   const uint64_t kk = static_cast<uint64_t>(p.top_k);
-  uint32_t rmask = 0;  // rows with any mass
-  float bmax[2];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    if (s < nr && !(f.aux[s].flags & kRowEmpty)) rmask |= 1u << s;
-    bmax[s] = f.aux[s].bmax;
-  }
   if (!rmask) return;
+  const float bmax[2] = {f.aux[0].bmax, f.aux[1].bmax};
   float ck[2];
   bool okk[2];
   {
@@ -2180,7 +2227,7 @@ __device__ __forceinline__ void resolve_top_k(const Params& p, FS& f, int nr, co
       for (int q = 0; q < kEPT; ++q) one[s][q] = eb[s][q] != 0u ? 1u : 0u;
     }
     const uint64_t k2[2] = {kk, kk};
-    select_entries<false>(f, rmask, k2, eb, one, false, ck, m1, okk, set1);
+    select_entries<false>(f, rmask, k2, eb, one, true, ck, m1, okk, set1);
   }
   uint32_t kmask = 0;  // rows whose k largest are entries
 #pragma unroll
@@ -2188,7 +2235,7 @@ __device__ __forceinline__ void resolve_top_k(const Params& p, FS& f, int nr, co
     if (((rmask >> s) & 1u) && okk[s] && ck[s] > bmax[s]) kmask |= 1u << s;
   }
   uint64_t mass[2] = {0u, 0u};
-  if (kmask) entries_mass2(f, kmask, ck, eb, ew, mass);
+  if (kmask) entries_mass2(f, kmask, ck, mass);
   // rows that still need a top-p select: those whose mass at and above ck
   // reaches thr, and those whose ck is not known to be the row's
   uint32_t pmask = 0;
@@ -2221,7 +2268,7 @@ __device__ __forceinline__ void resolve_top_k(const Params& p, FS& f, int nr, co
   }
   if (emask) {
     uint64_t em[2];
-    entries_mass2(f, emask, ck, eb, ew, em);
+    entries_mass2(f, emask, ck, em);
     if (emask & 1u) mass[0] = em[0];
     if (emask & 2u) mass[1] = em[1];
   }
@@ -2327,7 +2374,7 @@ __device__ __forceinline__ void pick_in_chunk(FS& f, int64_t c0, const uint64_t 
 template <class FS>
 __device__ __forceinline__ int64_t draw_list(const Params& p, FS& f, const uint64_t (&wl)[kEPT], float u,
                                              bool ordered) {
-  const int t = threadIdx.x;
+  const int t = thread_index();
   const uint32_t n = f.aux[0].n;
   uint32_t js;
   uint64_t rem;
@@ -2399,21 +2446,25 @@ __device__ __forceinline__ int64_t draw_list(const Params& p, FS& f, const uint6
 // chunk's mass by one wave, then the chunk holding the target by positions.
 template <int DT, bool kPair, typename WFn, class FS>
 __device__ __forceinline__ int64_t draw_dense(const Params& p, FS& f, int row0, int row1, float lo, float u, WFn wfn) {
-  const int t = threadIdx.x;
+  const int t = thread_index();
   const char* r0 = row_ptr(p, row0);
   const char* r1 = kPair ? row_ptr(p, row1) : nullptr;
   const uint32_t* bm = row_bitmap(p, row0);
   uint32_t* q = wave_queue(f);
   if (t == 0) f.token = 0;
-  each_chunk<DT, kPair, FS>(p, r0, r1, [&](int j, const ChunkData<DT>& c, const ChunkData<DT>& c1) {
+  uint64_t own = 0;  // of the chunk
+  each_piece<DT, kPair, FS>(p, r0, r1, bm, [&](int pq, const Piece<DT>& c, const Piece<DT>& c1) {
     constexpr int kBeside = kPair ? kPairX : kAlone;
-    uint64_t own = 0;
-    chunk_pass<DT, kBeside>(p, c, c1, bm, j, lo, __builtin_inff(), q, [&](const Batch<kBeside>& b) {
+    constexpr int kPer = Piece<DT>::kPerChunk;
+    piece_pass<DT, kBeside, true, FS>(p, c, c1, pq, lo, __builtin_inff(), q, [&](const Batch<kBeside, FS>& b) {
 #pragma unroll
       for (int k = 0; k < b.kN; ++k) own += b.valid[k] ? wfn(b.x[k], __uint_as_float(b.beside[k])) : 0u;
     });
-    own = wave_sum_u64(own);
-    if ((t & (kWave - 1)) == 0) f.csum[j] = own;
+    if (pq % kPer == kPer - 1 || (pq + 1) * Piece<DT>::kElems >= p.vocab) {
+      own = wave_sum_u64(own);
+      if ((t & (kWave - 1)) == 0) f.csum[pq / kPer] = own;
+      own = 0;
+    }
   });
   __syncthreads();
   pick_chunk(p, f, u);
@@ -2471,7 +2522,7 @@ __device__ __forceinline__ int64_t draw_target(const Params& p, FS& f, int row0,
 template <int DT, class FS>
 __device__ __forceinline__ int64_t draw_residual(const Params& p, FS& f, int row0, int row1, const RowK& K0, const RowK& K1,
                                  float u) {
-  const int t = threadIdx.x;
+  const int t = thread_index();
   const RowAux& a = f.aux[0];
   if (a.flags & kRowList) {
     const uint32_t n = a.n;
@@ -2544,8 +2595,8 @@ __device__ __forceinline__ int64_t draw_residual(const Params& p, FS& f, int row
   const uint32_t* bm = row_bitmap(p, row0);
   uint32_t* qu = wave_queue(f);
   uint64_t dsum = 0, psum = 0;
-  each_chunk<DT, true, FS>(p, row_ptr(p, row0), r1, [&](int j, const ChunkData<DT>& c, const ChunkData<DT>& c1) {
-    chunk_pass<DT, kPairX>(p, c, c1, bm, j, lo, __builtin_inff(), qu, [&](const Batch<kPairX>& b) {
+  each_piece<DT, true, FS>(p, row_ptr(p, row0), r1, bm, [&](int pq, const Piece<DT>& c, const Piece<DT>& c1) {
+    piece_pass<DT, kPairX, true, FS>(p, c, c1, pq, lo, __builtin_inff(), qu, [&](const Batch<kPairX, FS>& b) {
 #pragma unroll
       for (int k = 0; k < b.kN; ++k) {
         float P;
@@ -2646,17 +2697,22 @@ __device__ __forceinline__ void fin_unit(const Params& p, FS& f) {
       // a threshold of 0 (top_p < 2^-46) selects the largest p, as 1 does
       // whenever that p has a nonzero mass
       const uint64_t tf = fx46(tp);
-      thr[s] = tf > 0 ? tf : 1;
+      thr[s] = uniform(tf > 0 ? tf : 1);
     }
   }
   uint32_t eb[2][kEPT];
   uint64_t ew[2][kEPT];
-  place_entries(p, f, nr, sl, kTopK ? 0u : mask, eb, ew);
+  uint32_t rmask = 0;  // rows with any mass (with top-k, all of them are selected)
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    if (s < nr && !(f.aux[s].flags & kRowEmpty)) rmask |= 1u << s;
+  }
+  place_entries<kTopK>(p, f, nr, sl, kTopK ? rmask : mask, eb, ew);
   __syncthreads();
   RowK K[2];
-  for (int s = 0; s < 2; ++s) K[s] = RowK{f.aux[s < nr ? s : 0].mcmax, f.aux[s < nr ? s : 0].s, p.cd};
+  for (int s = 0; s < 2; ++s) K[s] = RowK{uniform(f.aux[s < nr ? s : 0].mcmax), uniform(f.aux[s < nr ? s : 0].s), p.cd};
   if constexpr (kTopK) {
-    resolve_top_k<DT>(p, f, nr, rows, K, mask, thr, eb, ew);
+    resolve_top_k<DT>(p, f, rows, K, rmask, mask, thr, eb, ew);
   } else {
     resolve_rows<DT, true>(p, f, rows, K, mask, thr, eb, ew, true);
   }
