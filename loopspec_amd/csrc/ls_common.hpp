@@ -48,7 +48,7 @@ __device__ __forceinline__ float vec_elem(const u32x4& d, int e) {
   }
 }
 
-// Scalar decode of element i of a row (unaligned fallback path).
+// Scalar decode of element i of a row (the elements beside a row's whole vectors).
 template <int DT>
 __device__ __forceinline__ float load_elem(const void* row, int64_t i) {
   if constexpr (DT == F32) {
