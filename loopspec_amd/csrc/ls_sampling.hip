@@ -1055,22 +1055,28 @@ struct FinShT {
 
 static_assert(sizeof(FinShT<10>) <= 80 * 1024, "two finaliser workgroups per CU");
 
-// A value every lane holds alike, in scalar registers (the whole-row passes keep
-// a unit's constants over code that needs every vector register).
+// With two finaliser workgroups per CU (128 registers) the whole-row passes need
+// every vector register, and what the set-up keeps for them would spill there.
+// uniform: a value every lane holds alike, in scalar registers. thread_index: the
+// thread's index, opaque to the compiler, so that addresses formed from it are
+// formed again where they are used. Where one workgroup has the CU both are left
+// to the compiler (C3 0.4 us shorter).
+template <class FS>
 __device__ __forceinline__ float uniform(float v) {
+  if constexpr (FS::kBits > 10) return v;
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }
+template <class FS>
 __device__ __forceinline__ uint64_t uniform(uint64_t v) {
+  if constexpr (FS::kBits > 10) return v;
   return pack_u32(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))),
                   static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32))));
 }
 
-// The thread's index, opaque to the compiler: addresses formed from it are
-// formed again where they are used, not kept in registers from one use to the
-// next over a whole row's select.
+template <class FS>
 __device__ __forceinline__ int thread_index() {
   int t = threadIdx.x;
-  asm volatile("" : "+v"(t));
+  if constexpr (FS::kBits <= 10) asm volatile("" : "+v"(t));
   return t;
 }
 
@@ -1351,7 +1357,7 @@ __device__ __forceinline__ void select_entries(FS& f, uint32_t mask, const uint6
                                                const uint32_t (&eb)[2][kEPT], const uint64_t (&ew)[2][kEPT],
                                                bool hist, float (&cut)[2], uint64_t (&mass)[2],
                                                bool (&ok)[2], bool (&set)[2]) {
-  const int t = thread_index(), lane = t & (kWave - 1), wid = t / kWave;
+  const int t = thread_index<FS>(), lane = t & (kWave - 1), wid = t / kWave;
   bool live[2] = {(mask & 1u) != 0, (mask & 2u) != 0};
   ok[0] = live[0];
   ok[1] = live[1];
@@ -1799,7 +1805,7 @@ __device__ __forceinline__ float lane_row_min(const Params& p, int row) {
 // Slot s's list entries 0 .. n - 1 selected for `thr` (kCount: by counts).
 template <bool kCount, class FS>
 __device__ __forceinline__ bool select_list(FS& f, int s, uint32_t n, uint64_t thr, float* cut, uint64_t* mass) {
-  const int t = thread_index();
+  const int t = thread_index<FS>();
   uint32_t eb[2][kEPT];
   uint64_t ew[2][kEPT];
 #pragma unroll
@@ -1896,7 +1902,7 @@ template <int DT, class FS>
 __device__ __forceinline__ bool select_window(const Params& p, FS& f, int s, int row, const RowK& K, uint64_t thr,
                                               float v_min, float* cut, uint64_t* mass) {
   constexpr int kStep = 4;
-  const int t = thread_index();
+  const int t = thread_index<FS>();
   uint32_t* fb = reinterpret_cast<uint32_t*>(f.u.bins[1]);
   uint64_t* bins = f.u.bins[0];
   const float inf = __builtin_inff();
@@ -1975,7 +1981,7 @@ __device__ __forceinline__ bool select_window(const Params& p, FS& f, int s, int
 template <int DT, bool kCount, class FS>
 __device__ __forceinline__ void select_row(const Params& p, FS& f, int s, int row, const RowK& K, uint64_t thr,
                                            float v_min, float* cut, uint64_t* mass) {
-  const int t = thread_index();
+  const int t = thread_index<FS>();
   if constexpr (!kCount) {
     if (select_window<DT>(p, f, s, row, K, thr, v_min, cut, mass)) return;
   }
@@ -2047,7 +2053,7 @@ __device__ __forceinline__ void select_row(const Params& p, FS& f, int s, int ro
 // (whose p becomes 0). False when they do not fit. Uses the draft hash's LDS.
 template <int DT, class FS>
 __device__ __forceinline__ bool refill_chunks(const Params& p, FS& f, int s, int row, const RowK& K, float c) {
-  const int t = thread_index(), lane = t & (kWave - 1);
+  const int t = thread_index<FS>(), lane = t & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(t / kWave);
   const char* rowp = row_ptr(p, row);
   const uint32_t* bm = row_bitmap(p, row);
@@ -2144,8 +2150,8 @@ __device__ __forceinline__ void resolve_rows(const Params& p, FS& f, const int (
       if ((late >> s) & 1u) store_row(f.aux[s], kRowFiltered | kRowList, cut[s], mass[s]);
     }
   }
-  const float g0 = uniform(ok[0] ? cut[0] : cutoff_guess(p, thr[0]));
-  const float g1 = uniform(ok[1] ? cut[1] : cutoff_guess(p, thr[1]));
+  const float g0 = uniform<FS>(ok[0] ? cut[0] : cutoff_guess(p, thr[0]));
+  const float g1 = uniform<FS>(ok[1] ? cut[1] : cutoff_guess(p, thr[1]));
 #pragma unroll 1
   for (int s = 0; s < 2; ++s) {
     if (!((whole >> s) & 1u)) continue;
@@ -2385,7 +2391,7 @@ __device__ __forceinline__ void pick_in_chunk(FS& f, int64_t c0, const uint64_t 
 template <class FS>
 __device__ __forceinline__ int64_t draw_list(const Params& p, FS& f, const uint64_t (&wl)[kEPT], float u,
                                              bool ordered) {
-  const int t = thread_index();
+  const int t = thread_index<FS>();
   const uint32_t n = f.aux[0].n;
   uint32_t js;
   uint64_t rem;
@@ -2457,7 +2463,7 @@ __device__ __forceinline__ int64_t draw_list(const Params& p, FS& f, const uint6
 // chunk's mass by one wave, then the chunk holding the target by positions.
 template <int DT, bool kPair, typename WFn, class FS>
 __device__ __forceinline__ int64_t draw_dense(const Params& p, FS& f, int row0, int row1, float lo, float u, WFn wfn) {
-  const int t = thread_index();
+  const int t = thread_index<FS>();
   const char* r0 = row_ptr(p, row0);
   const char* r1 = kPair ? row_ptr(p, row1) : nullptr;
   const uint32_t* bm = row_bitmap(p, row0);
@@ -2533,7 +2539,7 @@ __device__ __forceinline__ int64_t draw_target(const Params& p, FS& f, int row0,
 template <int DT, class FS>
 __device__ __forceinline__ int64_t draw_residual(const Params& p, FS& f, int row0, int row1, const RowK& K0, const RowK& K1,
                                  float u) {
-  const int t = thread_index();
+  const int t = thread_index<FS>();
   const RowAux& a = f.aux[0];
   if (a.flags & kRowList) {
     const uint32_t n = a.n;
@@ -2708,7 +2714,7 @@ __device__ __forceinline__ void fin_unit(const Params& p, FS& f) {
       // a threshold of 0 (top_p < 2^-46) selects the largest p, as 1 does
       // whenever that p has a nonzero mass
       const uint64_t tf = fx46(tp);
-      thr[s] = uniform(tf > 0 ? tf : 1);
+      thr[s] = uniform<FS>(tf > 0 ? tf : 1);
     }
   }
   uint32_t eb[2][kEPT];
@@ -2721,7 +2727,7 @@ __device__ __forceinline__ void fin_unit(const Params& p, FS& f) {
   place_entries<kTopK>(p, f, nr, sl, kTopK ? rmask : mask, eb, ew);
   __syncthreads();
   RowK K[2];
-  for (int s = 0; s < 2; ++s) K[s] = RowK{uniform(f.aux[s < nr ? s : 0].mcmax), uniform(f.aux[s < nr ? s : 0].s), p.cd};
+  for (int s = 0; s < 2; ++s) K[s] = RowK{uniform<FS>(f.aux[s < nr ? s : 0].mcmax), uniform<FS>(f.aux[s < nr ? s : 0].s), p.cd};
   if constexpr (kTopK) {
     resolve_top_k<DT>(p, f, rows, K, rmask, mask, thr, eb, ew);
   } else {
