@@ -134,9 +134,17 @@ def check(status: int) -> None:
     raise RuntimeError(msg)
 
 
+_entries: dict[str, object] = {}
+
+
 def call(name: str, *args) -> None:
     """Invoke a status-returning entry point and raise on failure."""
-    check(getattr(load(), name)(*args))
+    fn = _entries.get(name)
+    if fn is None:
+        fn = _entries[name] = getattr(load(), name)
+    status = fn(*args)
+    if status != LS_OK:
+        check(status)
 
 
 @functools.lru_cache(maxsize=1024)

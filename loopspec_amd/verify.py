@@ -208,21 +208,21 @@ def greedy_verify(
             raise ValueError("draft_tokens must be int64 [B, k]")
         draft_tokens = draft_tokens.contiguous()
         d_ptr, d_bs, d_ps, tok_ptr = None, 0, 0, draft_tokens.data_ptr()
+    # a step is a few microseconds of kernel: only what the caller passed is checked
     if accept_len is None:
         accept_len = torch.empty(batch, dtype=torch.int32, device=dev)
+    elif accept_len.shape != (batch,) or accept_len.dtype != torch.int32 or not accept_len.is_contiguous():
+        raise ValueError("accept_len must be contiguous int32 [B]")
     if tokens is None:
         tokens = torch.empty((batch, kp1), dtype=torch.int64, device=dev)
-    if accept_len.shape != (batch,) or accept_len.dtype != torch.int32 or not accept_len.is_contiguous():
-        raise ValueError("accept_len must be contiguous int32 [B]")
-    if tokens.shape != (batch, kp1) or tokens.dtype != torch.int64 or not tokens.is_contiguous():
+    elif tokens.shape != (batch, kp1) or tokens.dtype != torch.int64 or not tokens.is_contiguous():
         raise ValueError("tokens must be contiguous int64 [B, k+1]")
     if row_argmax is not None and (
         row_argmax.shape != (batch, 2 * k + 1) or row_argmax.dtype != torch.int64 or not row_argmax.is_contiguous()
     ):
         raise ValueError("row_argmax must be contiguous int64 [B, 2k+1]")
-    nbytes = _lib.query("ls_greedy_verify_workspace", batch, k, vocab)
-    ws = workspace if workspace is not None else _lib.WORKSPACE.get(dev, nbytes, "greedy",
-                                                                     keep=_status_header_bytes())
+    ws = workspace if workspace is not None else _lib.WORKSPACE.get(
+        dev, _lib.query("ls_greedy_verify_workspace", batch, k, vocab), "greedy", keep=_status_header_bytes())
     _lib.call(
         "ls_greedy_verify",
         target_logits.data_ptr(), target_logits.stride(0), target_logits.stride(1),
