@@ -3217,7 +3217,15 @@ int ls_filter_logits(const void* logits, int64_t row_stride, int dtype, int64_t 
   // Without the unfiltered rows, a filtered row is zeros but for its support,
   // which the finaliser holds: no second pass over the logits (64 rows, V 49152
   // f32, top-p 0.7: 27.0 -> 23.3 us a call; 200 rows, V 128256 bf16: 106 -> 57).
-  p.zero_out = filtered_out && !probs_out && p.vec_out && (top_p < 1.0f || p.top_k);
+  // Not where the output overlaps the logits, which the finaliser may read again.
+  auto disjoint = [&](const void* x, int64_t xs, int64_t xb, const void* y, int64_t ys, int64_t yb) {
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
+    const uintptr_t x1 = x0 + static_cast<uintptr_t>(((rows - 1) * xs + vocab) * xb);
+    const uintptr_t y1 = y0 + static_cast<uintptr_t>(((rows - 1) * ys + vocab) * yb);
+    return x1 <= y0 || y1 <= x0;
+  };
+  p.zero_out = filtered_out && !probs_out && p.vec_out && (top_p < 1.0f || p.top_k) && row_stride >= 0 &&
+               filtered_stride >= vocab && disjoint(logits, row_stride, eb, filtered_out, filtered_stride, 4);
   const Layout l = ws_layout(rows, 0, rows, p.nch);
   if (!workspace || ws_bytes < l.total) return fail(LS_ERR_VALUE, "filter_logits: workspace too small");
   bind_workspace(p, workspace, l);

@@ -30,3 +30,17 @@ def test_filtered_rows_at_any_stride(gpu, vocab, dtype, pad, top_p, top_k):
     torch.cuda.synchronize()
     assert torch.equal(out[:rows, :vocab].view(torch.int32), both["filtered"].view(torch.int32))
     assert bool((out[:rows, vocab:] == -3.0).all()) and bool((out[rows] == -3.0).all())
+
+
+@pytest.mark.parametrize("top_p", [0.6, 0.97])
+def test_filtered_rows_over_their_logits(gpu, top_p):
+    """The filtered rows written over float32 logits (the support re-read included)."""
+    rows, vocab = 3, 20000
+    x = (torch.randn(rows, vocab, generator=torch.Generator().manual_seed(1)) * 3).to(gpu)
+    announce(f"filter in place p={top_p}")
+    want = verify.filter_logits(x, 1.0, top_p)["filtered"]
+    ws = torch.zeros(_lib.query("ls_filter_logits_workspace", rows, vocab), dtype=torch.uint8, device=gpu)
+    _lib.call("ls_filter_logits", x.data_ptr(), x.stride(0), _lib.dtype_code(x), rows, vocab, 1.0, top_p, None, 0,
+              None, 0, x.data_ptr(), x.stride(0), None, None, ws.data_ptr(), ws.numel(), _lib.stream(gpu))
+    torch.cuda.synchronize()
+    assert torch.equal(x.view(torch.int32), want.view(torch.int32))
