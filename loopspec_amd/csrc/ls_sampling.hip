@@ -1541,19 +1541,31 @@ __device__ __forceinline__ void select_entries(FS& f, uint32_t mask, const uint6
 // ---------------------------------------------------------------------------
 constexpr int kQueue = kHash / kFNW;  // words of LDS (the draft hash's) a wave queues logits in
 
-// A logit no element with p >= v lies below (slack for the roundings of p's
-// exponent, polynomial and division: together under 2^-16 octaves).
+// Logits that bracket an element's p without forming it. p = RN(e / S) with
+// e = RN(E), E the unrounded power of two: a relative rounding moves p by 2^-24,
+// but where p or e is subnormal it moves it by up to half of 2^-149, any number
+// of octaves of the smallest ones. So p >= v means e / S >= v - h and
+// E >= S (v - h) - h with h = 2^-150, and p < v means e / S <= v - h and
+// E <= S (v - h) + h (both exact in binary64 where h matters). The relative
+// roundings (of p, of E's polynomial and exponent: under 2^-16 octaves) are
+// covered by 2^-10 octaves of slack.
+constexpr double kHalfUlp0 = 0x1p-150;
+constexpr double kLogSlack = 0x1p-10;
+
+// A logit no element with p >= v lies below.
 __device__ __forceinline__ float x_floor(const RowK& K, float v) {
-  if (!(v > 0.0f)) return -__builtin_inff();
-  const double t = log2(static_cast<double>(v) * static_cast<double>(K.s)) - 1.0e-3;
-  const float x = static_cast<float>((t + static_cast<double>(K.mcmax)) / K.cd);
+  const double s = static_cast<double>(K.s);
+  const double e = __builtin_fma(s, static_cast<double>(v) - kHalfUlp0, -kHalfUlp0);
+  if (!(e > 0.0)) return -__builtin_inff();
+  const float x = static_cast<float>((log2(e) - kLogSlack + static_cast<double>(K.mcmax)) / K.cd);
   return -next_up(-x);
 }
 
-// A logit no element with p < v lies above.
+// A logit no element with p < v lies above (v > 0).
 __device__ __forceinline__ float x_ceil(const RowK& K, float v) {
-  const double t = log2(static_cast<double>(v) * static_cast<double>(K.s)) + 1.0e-3;
-  return next_up(static_cast<float>((t + static_cast<double>(K.mcmax)) / K.cd));
+  const double s = static_cast<double>(K.s);
+  const double e = __builtin_fma(s, static_cast<double>(v) - kHalfUlp0, kHalfUlp0);
+  return next_up(static_cast<float>((log2(e) + kLogSlack + static_cast<double>(K.mcmax)) / K.cd));
 }
 
 // Orders a wave's own LDS traffic (the LDS serves a wave in order; this keeps

@@ -84,3 +84,23 @@ def test_filter_and_sample_large_support_edges(gpu, kind, top_p, top_k):
         assert res["cutoff"][r].item() == want.cutoff, r
         assert res["mass"][r].item() == nm.mass_to_f32(want.mass_fx), r
         assert got[r].item() == osmp.categorical_pick(want.P, u[r].item()), r
+
+
+@pytest.mark.parametrize("ulps", [256, 512])
+@pytest.mark.parametrize("ties", [1500, 3000])  # inside the list's 2048, and past it
+def test_top_k_at_a_subnormal_plateau(gpu, ulps, ties):
+    """The k-th largest p is a plateau at 256 or 512 * 2^-149, the first value of a
+    digit, whose logits' powers of two lie half of 2^-149 below it."""
+    v = 16392
+    x = np.full((2, v), -1000.0, dtype=np.float32)
+    x[:, 0] = 0.0
+    x[:, 3:3 + 5 * ties:5] = np.float32(np.log((ulps - 0.4) * 2.0 ** -149))
+    announce(f"subnormal plateau ulps={ulps} ties={ties}")
+    res = verify.filter_logits(torch.from_numpy(x).to(gpu), 1.0, 1.0, top_k=1000)
+    torch.cuda.synchronize()
+    want = osmp.filter_row(osmp.process_logits(x[0], 1.0, epv=4), 1.0, 1000)
+    assert want.cutoff == np.float32(ulps * 2.0 ** -149)
+    for r in range(2):
+        assert res["cutoff"][r].item() == want.cutoff, r
+        assert np.array_equal(res["filtered"][r].cpu().numpy(), want.P), r
+        assert res["mass"][r].item() == nm.mass_to_f32(want.mass_fx), r
