@@ -55,6 +55,7 @@ constexpr int kLmMaxRows = 320;                // rows per workgroup: 64 MT for 
 constexpr int kLmBN = 2 * kLmColsPerWave;      // 192 columns per workgroup
 constexpr int kLmKB = 64;                      // k per LDS block
 constexpr int kXcds = 8;
+constexpr int kGridXLog2 = 22;                 // workgroups along x at most (see head_grid)
 constexpr int kLmRowBytes = kLmKB * 2;         // 128 bytes of a row's k-block
 constexpr int kLmBRounds = 3;  // 24 x 1 KB per B block over 8 waves
 
@@ -96,6 +97,13 @@ __device__ __forceinline__ void dma16_stream(const void* src, uint32_t lds) {
   asm volatile("global_load_lds_dwordx4 %0, off nt" : : "v"(src), "{m0}"(lds) : "memory");
 }
 
+// A head workgroup's index. A launch dimension holds fewer than 2^32 lanes, so
+// workgroups past the first 2^22 go along y; in dispatch order the index still
+// counts up by one.
+__device__ __forceinline__ int head_block() {
+  return static_cast<int>(blockIdx.x + (blockIdx.y << kGridXLog2));
+}
+
 // Byte offset of 16-byte chunk c of row r in an A block.
 __device__ __forceinline__ int a_off(int r, int c) { return r * kLmRowBytes + ((c ^ (r & 7)) << 4); }
 
@@ -123,13 +131,13 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
   // the whole weight was streamed once per row block: 1260 us against 1120 at
   // M 1280, H 4096, V 128256. Giving each XCD a run of column blocks of one row
   // block, for its hidden rows to stay in L2, measured 1160.)
-  int m_blk = 0, nblk = static_cast<int>(blockIdx.x);
+  int m_blk = 0, nblk = head_block();
   if (p.mblk > 1) {
     const int xcd = nblk & (kXcds - 1), at = nblk / kXcds;
     m_blk = at % p.mblk;
     nblk = at / p.mblk * kXcds + xcd;
-    if (nblk >= p.nblk) return;
   }
+  if (nblk >= p.nblk) return;
   const int64_t m_base = static_cast<int64_t>(m_blk) * kBM;
   const int64_t n_base = static_cast<int64_t>(nblk) * kLmBN;
   const int nkb = static_cast<int>(p.H / kLmKB);
@@ -348,7 +356,8 @@ __global__ __launch_bounds__(kLrLanes) void lm_head_rows_kernel(const LmParams p
   __shared__ uint64_t keys[kRows][kLrWaves];
   const int t = threadIdx.x, lane = t & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(t / kWave);
-  const int nblk = static_cast<int>(blockIdx.x);
+  const int nblk = head_block();
+  if (nblk >= p.nblk) return;
   const int64_t n_base = static_cast<int64_t>(nblk) * kLmBN;
   const int nkb = static_cast<int>(p.H / kLmKB);
   const int64_t col = n_base + w * 16 + (lane & 15);  // of this lane's accumulators
@@ -598,12 +607,23 @@ uint64_t ls_lm_head_argmax_workspace(int64_t rows, int64_t vocab) {
 
 namespace {
 
+// Column blocks as launched: with several row blocks in groups of kXcds, each
+// with its row blocks (see lm_head_kernel).
+int64_t launched_cols(int64_t nblk, int64_t mblk) { return mblk > 1 ? (nblk + kXcds - 1) / kXcds * kXcds : nblk; }
+
+// head_block's grid of n workgroups; those past n leave at once.
+dim3 head_grid(int64_t n) {
+  constexpr int64_t kMaxX = int64_t{1} << kGridXLog2;
+  static_assert(kMaxX * kLrLanes < (int64_t{1} << 32) && kMaxX * kLmLanes < (int64_t{1} << 32), "lanes along x");
+  return n <= kMaxX ? dim3(static_cast<unsigned>(n)) : dim3(kMaxX, static_cast<unsigned>((n + kMaxX - 1) / kMaxX));
+}
+
 // The kernel of a head call: a rule on the rows alone, so that every entry
 // point forms a row's logits by the same products in the same order.
 template <int EPI>
 void launch_head(const LmParams& p, hipStream_t st) {
   if (p.M <= 32) {
-    const dim3 grid(static_cast<unsigned>(p.nblk));
+    const dim3 grid = head_grid(p.nblk);
     if (p.M <= 16) {
       hipLaunchKernelGGL((lm_head_rows_kernel<1, EPI>), grid, dim3(kLrLanes), 0, st, p);
     } else {
@@ -611,9 +631,7 @@ void launch_head(const LmParams& p, hipStream_t st) {
     }
     return;
   }
-  // column blocks in groups of kXcds, each with its row blocks (see the kernel)
-  const int cols = p.mblk > 1 ? (p.nblk + kXcds - 1) / kXcds * kXcds : p.nblk;
-  const dim3 grid(static_cast<unsigned>(cols) * static_cast<unsigned>(p.mblk));
+  const dim3 grid = head_grid(launched_cols(p.nblk, p.mblk) * p.mblk);
   const int64_t rows = (p.M + p.mblk - 1) / p.mblk;  // per row block
   if (rows <= 64) {
     hipLaunchKernelGGL((lm_head_kernel<1, EPI>), grid, dim3(kLmLanes), 0, st, p);
@@ -647,6 +665,9 @@ int lm_head_launch(const char* what, const void* hidden, int64_t hidden_stride, 
   const int64_t nblk = (vocab + kLmBN - 1) / kLmBN;
   const int64_t mblk = (rows + kLmMaxRows - 1) / kLmMaxRows;
   if (mblk > 65535) return fail(LS_ERR_VALUE, w + ": too many rows");
+  // (their keys or logits would fill hundreds of GB)
+  if (launched_cols(nblk, mblk) * mblk > 0x7fffffffLL - (1LL << kGridXLog2))
+    return fail(LS_ERR_VALUE, w + ": rows x vocab too large");
   if (epi == kLmKeys && (workspace == nullptr || ws_bytes < ls_lm_head_argmax_workspace(rows, vocab)))
     return fail(LS_ERR_VALUE, w + ": workspace too small");
   if (epi != kLmKeys && (logits == nullptr || logits_stride < vocab))

@@ -5,7 +5,7 @@ column counts around a block."""
 import pytest
 import torch
 
-from loopspec_amd import verify
+from loopspec_amd import _lib, verify
 from tests.conftest import announce
 from tests.test_lm_head_gpu import check, make, reference
 
@@ -29,3 +29,24 @@ def test_lm_head_rows(gpu, rows, hidden_size, vocab):
     assert torch.equal(f32.argmax(-1), ids)
     # nothing is written past the rows and columns asked for
     assert bool((out[rows] == 7.0).all()) and bool((out[:, vocab:] == 7.0).all())
+
+
+def test_lm_head_more_workgroups_than_one_launch_dimension(gpu):
+    """10,485,800 rows at 256 column blocks: 2^23 workgroups of 512 lanes and more
+    than 2^32 lanes. The rows repeat 97 others, whose period meets every place of a
+    row block, so the ids must repeat theirs."""
+    period, rows, hidden_size, vocab = 97, 10_485_800, 64, 49152
+    hidden, weight = make(period, hidden_size, vocab, 5)
+    announce(f"lm_head M={rows} H={hidden_size} V={vocab}")
+    h, w = hidden.to(gpu), weight.to(gpu)
+    want = verify.lm_head_argmax(h, w)
+    check(want.cpu().numpy(), *reference(hidden, weight))
+    many = h.repeat(-(-rows // period), 1)[:rows]
+    out = torch.empty(rows, dtype=torch.int64, device=gpu)
+    ws = torch.empty(_lib.query("ls_lm_head_argmax_workspace", rows, vocab), dtype=torch.uint8, device=gpu)
+    _lib.call("ls_lm_head_argmax", many.data_ptr(), many.stride(0), w.data_ptr(), w.stride(0), _lib.dtype_code(many),
+              rows, hidden_size, vocab, out.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream(gpu))
+    torch.cuda.synchronize()
+    assert torch.equal(out, want.repeat(-(-rows // period))[:rows])
+    del ws
+    torch.cuda.empty_cache()
