@@ -1982,8 +1982,8 @@ __device__ __forceinline__ bool select_window(const Params& p, FS& f, int s, int
 // Exact cutoff of a whole row: c = max{v : sum over the row's p >= v of
 // fx46(p) >= thr} (kCount: every element weighs 1, so thr = k gives the k-th
 // largest p, duplicates counted), *mass the sum at and above it. v_min: a p the
-// cutoff probably does not lie below. Masses take select_window's two passes
-// first. What those leave undecided, and counts, take radix rounds on the bits
+// cutoff does not lie below (masses: probably not). Masses take select_window's
+// two passes first. What those leave undecided, and counts, take radix rounds on the bits
 // of p as in select_entries: a pass over the row bins the masses of the current
 // digit, the crossing digit's elements are gathered by a second pass into slot
 // s's entries and finished by select_entries when they fit, else the next digit
@@ -1999,7 +1999,7 @@ __device__ __forceinline__ void select_row(const Params& p, FS& f, int s, int ro
   }
   uint64_t* bins = f.u.bins[0];
   const float inf = __builtin_inff();
-  float lo = -inf, hi = inf;
+  float lo = kCount ? x_floor(K, v_min) : -inf, hi = inf;
   uint32_t prefix = 0;
   uint64_t above = 0;
 #pragma unroll 1
@@ -2133,9 +2133,9 @@ __device__ __forceinline__ void store_row(RowAux& a, uint32_t flags, float cut, 
 // state. A select over the entries is the row's when its cutoff lies above
 // every chunk's non-candidate bound. Otherwise that cutoff, when the entries
 // hold thr, is a lower bound of the row's: the chunks whose bound reaches it
-// are re-read (kRefill) and the entries selected again; a row they do not fit,
+// are re-read and the entries selected again; a row they do not fit,
 // or whose entries hold less than thr, is selected whole.
-template <int DT, bool kRefill, class FS>
+template <int DT, class FS>
 __device__ __forceinline__ void resolve_rows(const Params& p, FS& f, const int (&rows)[2], const RowK (&K)[2], uint32_t mask,
                                             const uint64_t (&thr)[2], const uint32_t (&eb)[2][kEPT],
                                             const uint64_t (&ew)[2][kEPT], bool hist) {
@@ -2174,7 +2174,7 @@ __device__ __forceinline__ void resolve_rows(const Params& p, FS& f, const int (
     float c;
     uint64_t m;
     uint32_t flags = kRowFiltered;
-    if (kRefill && (s == 0 ? ok[0] : ok[1]) && refill_chunks<DT>(p, f, s, row, Ks, g) &&
+    if ((s == 0 ? ok[0] : ok[1]) && refill_chunks<DT>(p, f, s, row, Ks, g) &&
         select_list<false>(f, s, f.aux[s].n, th, &c, &m)) {
       flags |= kRowList | kRowRefilled;
     } else {
@@ -2206,6 +2206,37 @@ __device__ __forceinline__ void entries_mass2(FS& f, uint32_t mask, const float 
   __syncthreads();
 }
 
+// sum_{p >= c} fx46(p) over slot s's list entries 0 .. n - 1 (kCount: the number of them).
+template <bool kCount, class FS>
+__device__ __forceinline__ uint64_t list_mass(FS& f, int s, uint32_t n, float c) {
+  uint64_t own = 0;
+  for (uint32_t e = threadIdx.x; e < n; e += kFW) {
+    const float v = __uint_as_float(f.ent[s].pbits[e]);
+    if (v >= c) own += kCount ? uint64_t{1} : fx46(v);
+  }
+  const uint64_t tot = block_sum(own, f.red[2]);
+  __syncthreads();
+  return tot;
+}
+
+// The elements p >= c of a whole row into slot s's entries, in no order and
+// without their indices; returns their number (past kRowCap they are counted only).
+template <int DT, class FS>
+__device__ __forceinline__ uint32_t gather_row(const Params& p, FS& f, int s, int row, const RowK& K, float c) {
+  __syncthreads();  // earlier reads of the list
+  if (threadIdx.x == 0) f.gcount[s] = 0;
+  __syncthreads();
+  row_pass<DT>(p, f, row, x_floor(K, c), __builtin_inff(), [&](const Batch<kAlone, FS>& b) {
+#pragma unroll
+    for (int k = 0; k < b.kN; ++k) {
+      const float v = pval(K, b.x[k]);
+      list_append<false>(f, s, &f.gcount[s], b.valid[k] && v >= c, __float_as_uint(v), 0u);
+    }
+  });
+  __syncthreads();
+  return f.gcount[s];
+}
+
 // sum_{p >= c} fx46(p) over a whole row.
 template <int DT, class FS>
 __device__ __forceinline__ uint64_t row_mass(const Params& p, FS& f, int row, const RowK& K, float c) {
@@ -2227,21 +2258,24 @@ __device__ __forceinline__ uint64_t row_mass(const Params& p, FS& f, int row, co
 // largest alone for the rows not in `mask` (top_p = 1) -- with ties kept and
 // one renormalisation over {p >= cutoff}. rmask: the rows with any mass, whose
 // entries are counted in the bins already. The k-th largest ck of the entries
-// comes first, by a select by counts over both rows. Above every chunk's
-// non-candidate bound it is the row's, and every element at or above it is an
-// entry, so the top-p cutoff cp is decided there too: the entries' mass at and
-// above ck falls short of thr exactly when cp < ck (the cutoff is ck), and
-// otherwise cp >= ck is the entries' own. So a row whose top-p support is far
-// larger than its candidates needs no pass over the row when its k largest are
-// among them (one sequence, k = 4, V = 32000, T 0.8, top_p 0.95, top_k 50: the
-// finaliser took 25 to 164 us with top-p resolved first). Rows whose k largest
-// are not all candidates take their top-p cutoff first: a list-mode row's other
-// elements lie below cp, so its cutoff is max(ck, cp) over the entries; any
-// other row is selected by counts over the whole row.
+// comes first, by a select by counts over both rows. Above every chunk's non-candidate bound it is the row's, and every element at or
+// above it is an entry, so the top-p cutoff cp is decided there too: the
+// entries' mass at and above ck falls short of thr exactly when cp < ck (the
+// cutoff is ck), and otherwise cp >= ck is the entries' own. So a row whose
+// top-p support is far larger than its candidates needs no pass over the row
+// when its k largest are among them (one sequence, k = 4, V = 32000, T 0.8,
+// top_p 0.95, top_k 50: the finaliser took 25 to 164 us with top-p resolved
+// first). Rows whose k largest are not all candidates take their top-p cutoff
+// first, and keep it when no more than k elements reach it. Otherwise the
+// k-th largest of those elements is the cutoff: of the entries, counted again
+// where chunks were re-read into them or the row's support was gathered, or of
+// the whole row (B 64, k 2, V 49152
+// f32, T 0.7, top_p 0.95, top_k 1000, chunks re-read: 140 us a call with the
+// whole row selected twice instead).
 template <int DT, class FS>
 __device__ __forceinline__ void resolve_top_k(const Params& p, FS& f, const int (&rows)[2], const RowK (&K)[2],
-                                              uint32_t rmask, uint32_t mask, const uint64_t (&thr)[2], const uint32_t (&eb)[2][kEPT],
-                                              const uint64_t (&ew)[2][kEPT]) {
+                                              uint32_t rmask, uint32_t mask, const uint64_t (&thr)[2],
+                                              const uint32_t (&eb)[2][kEPT], const uint64_t (&ew)[2][kEPT]) {
   const uint64_t kk = static_cast<uint64_t>(p.top_k);
   if (!rmask) return;
   const float bmax[2] = {f.aux[0].bmax, f.aux[1].bmax};
@@ -2272,28 +2306,35 @@ __device__ __forceinline__ void resolve_top_k(const Params& p, FS& f, const int 
   for (int s = 0; s < 2; ++s) {
     if (((mask >> s) & 1u) && !(((kmask >> s) & 1u) && mass[s] < thr[s])) pmask |= 1u << s;
   }
-  if (pmask) resolve_rows<DT, false>(p, f, rows, K, pmask, thr, eb, ew, false);
-  uint32_t fl[2];
-  float cp[2];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    fl[s] = f.aux[s].flags;
-    cp[s] = ((pmask >> s) & 1u) ? f.aux[s].cut : 0.0f;
-  }
+  if (pmask) resolve_rows<DT>(p, f, rows, K, pmask, thr, eb, ew, false);
   uint32_t store = 0, emask = 0, whole = 0;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     if (!((rmask >> s) & 1u)) continue;
     if ((kmask >> s) & 1u) {
       if (!((pmask >> s) & 1u)) store |= 1u << s;  // else cp >= ck: as resolved
-    } else if (((pmask >> s) & 1u) && (fl[s] & kRowList)) {
-      if (okk[s] && ck[s] > cp[s]) {
-        store |= 1u << s;
-        emask |= 1u << s;
-      }
+    } else if (((pmask >> s) & 1u) && (f.aux[s].flags & kRowList)) {
+      if (okk[s] && ck[s] > f.aux[s].cut) emask |= 1u << s;
     } else {
       whole |= 1u << s;
     }
+  }
+#pragma unroll 1
+  for (int s = 0; s < 2; ++s) {
+    // re-read rows: the elements at and above cp in the list, and where they
+    // are more than k the k-th largest of the list (its dead entries count at
+    // p = 0, below any cutoff)
+    if (!((pmask >> s) & 1u) || !(f.aux[s].flags & kRowRefilled)) continue;
+    const uint32_t n = f.aux[s].n;
+    const float cp = f.aux[s].cut;
+    emask &= ~(1u << s);
+    if (list_mass<true>(f, s, n, cp) <= kk) continue;
+    float c;
+    uint64_t m;
+    select_list<true>(f, s, n, kk, &c, &m);
+    if (c > cp) emask |= 1u << s;
+    if (s == 0) ck[0] = c;
+    else ck[1] = c;
   }
   if (emask) {
     uint64_t em[2];
@@ -2305,7 +2346,8 @@ __device__ __forceinline__ void resolve_top_k(const Params& p, FS& f, const int 
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      if ((store >> s) & 1u) store_row(f.aux[s], kRowFiltered | kRowList, ck[s], mass[s]);
+      if (((store | emask) >> s) & 1u)
+        store_row(f.aux[s], kRowFiltered | kRowList | (f.aux[s].flags & kRowRefilled), ck[s], mass[s]);
     }
   }
 #pragma unroll 1
@@ -2314,12 +2356,23 @@ __device__ __forceinline__ void resolve_top_k(const Params& p, FS& f, const int 
     // the k-th largest of the whole row by passes over it
     const int row = s == 0 ? rows[0] : rows[1];
     const RowK Ks = s == 0 ? K[0] : K[1];
-    const float lower = s == 0 ? cp[0] : cp[1];
+    const float lower = ((pmask >> s) & 1u) ? uniform<FS>(f.aux[s].cut) : 0.0f;
     float c;
     uint64_t m;
-    select_row<DT, true>(p, f, s, row, Ks, kk, 0.0f, &c, &m);
-    c = c > lower ? c : lower;
-    m = row_mass<DT>(p, f, row, Ks, c);
+    bool listed = false;  // the elements at and above cp, all of them
+    if (lower > 0.0f) {
+      const uint32_t n = gather_row<DT>(p, f, s, row, Ks, lower);
+      if (n <= kk) continue;
+      listed = n <= static_cast<uint32_t>(kRowCap);
+      if (listed) {
+        select_list<true>(f, s, n, kk, &c, &m);
+        m = list_mass<false>(f, s, n, c);
+      }
+    }
+    if (!listed) {
+      select_row<DT, true>(p, f, s, row, Ks, kk, lower, &c, &m);
+      m = row_mass<DT>(p, f, row, Ks, c);
+    }
     if (threadIdx.x == 0) store_row(f.aux[s], kRowFiltered, c, m);
   }
   __syncthreads();
@@ -2743,7 +2796,7 @@ __device__ __forceinline__ void fin_unit(const Params& p, FS& f) {
   if constexpr (kTopK) {
     resolve_top_k<DT>(p, f, rows, K, rmask, mask, thr, eb, ew);
   } else {
-    resolve_rows<DT, true>(p, f, rows, K, mask, thr, eb, ew, true);
+    resolve_rows<DT>(p, f, rows, K, mask, thr, eb, ew, true);
   }
 
   if (p.mode == kModeSpec) {

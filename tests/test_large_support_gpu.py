@@ -10,6 +10,7 @@ import torch
 from oracle import numerics as nm
 from oracle import sampling as osmp
 from loopspec_amd import philox, verify, workloads
+from tests import candidates
 from tests.conftest import announce
 from tests.test_sweep_gpu import epv_of, histories, oracle_drafts
 
@@ -104,3 +105,32 @@ def test_top_k_at_a_subnormal_plateau(gpu, ulps, ties):
         assert res["cutoff"][r].item() == want.cutoff, r
         assert np.array_equal(res["filtered"][r].cpu().numpy(), want.P), r
         assert res["mass"][r].item() == nm.mass_to_f32(want.mass_fx), r
+
+
+@pytest.mark.parametrize("rows", [2, 300])  # one finaliser workgroup per CU, and two
+@pytest.mark.parametrize("dtype,penalty", [(F32, 1.0), (BF16, 1.0), (F32, 1.3)])
+@pytest.mark.parametrize("top_k", [0, 40, 50, 51, 150, 151, 700])  # 50 tokens at 6.0, then 100 ties at 5.0
+def test_re_read_chunks_with_top_k(gpu, rows, dtype, penalty, top_k):
+    """Rows with a chunk that keeps no candidates: it is re-read, and the k-th
+    largest is known only from the re-read list (above, at and below the top-p cutoff)."""
+    row, top_p = candidates.path_rows()["refill"]
+    x = torch.from_numpy(row).to(dtype)
+    assert candidates.row_path(x.float().numpy(), top_p, epv=epv_of(dtype)) == "refill"
+    hist = np.flatnonzero(row == 6.0)[::3].astype(np.int32)
+    batch = torch.stack([x, x.flip(0)]).repeat(rows // 2, 1)
+    hists = [hist, (len(row) - 1 - hist).astype(np.int32)]
+    u = torch.from_numpy(philox.uniforms((rows,), seed=top_k))
+    announce(f"re-read rows={rows} {dtype} pen={penalty} k={top_k}")
+    pen = {} if penalty == 1.0 else {"penalty": penalty, "history": torch.from_numpy(np.stack(hists)).repeat(rows // 2, 1).to(gpu)}
+    got = verify.sample_logits(batch.to(gpu), u.to(gpu), 1.0, top_p, top_k=top_k, **pen)
+    res = verify.filter_logits(batch.to(gpu), 1.0, top_p, top_k=top_k) if not pen else None
+    torch.cuda.synchronize()
+    want = [osmp.filter_row(osmp.process_logits(batch[r].float().numpy(), 1.0, penalty, hists[r] if pen else None,
+                                                epv_of(dtype)), top_p, top_k) for r in range(2)]
+    assert got.cpu().tolist() == [osmp.categorical_pick(want[r % 2].P, u[r].item()) for r in range(rows)]
+    for r in range(rows if res else 0):
+        assert res["cutoff"][r].item() == want[r % 2].cutoff, r
+        assert res["mass"][r].item() == nm.mass_to_f32(want[r % 2].mass_fx), r
+    if res:
+        P = torch.from_numpy(np.stack([w.P for w in want])).to(gpu).repeat(rows // 2, 1)
+        assert torch.equal(res["filtered"], P)
