@@ -1596,15 +1596,17 @@ struct Piece {
   u32x4 bits;
 };
 
-// Piece q of a row (element q * kElems on).
+// Piece q of a row (element q * kElems on), or its vectors u0 .. u1 - 1 only.
 template <int DT>
-__device__ __forceinline__ void load_piece(const Params& p, const char* rowp, const uint32_t* bm, int q, Piece<DT>& c) {
+__device__ __forceinline__ void load_piece(const Params& p, const char* rowp, const uint32_t* bm, int q, Piece<DT>& c,
+                                           int u0 = 0, int u1 = Piece<DT>::kVecs) {
   constexpr int EPV = Elem<DT>::kPerVec;
   const int lane = threadIdx.x & (kWave - 1);
   const int v0 = q * Piece<DT>::kElems / EPV, nv = p.vocab / EPV;
   const u32x4* src = reinterpret_cast<const u32x4*>(rowp);
 #pragma unroll
   for (int u = 0; u < Piece<DT>::kVecs; ++u) {
+    if (u < u0 || u >= u1) continue;
     const int at = v0 + u * kWave + lane, v = at < nv ? at : nv - 1;
     const u32x4 x = src[v];
 #pragma unroll
@@ -1653,27 +1655,34 @@ struct Batch {
   bool valid[kN];
 };
 
+// A piece as piece_pass takes it: kStep elements of every lane, kSteps times.
+template <int DT, int kBeside>
+struct Pass {
+  static constexpr int kStep = kBeside == kAlone ? 4 : 2;  // elements between drains
+  static constexpr int kSteps = Piece<DT>::kElems / kWave / kStep;
+};
+
 // One wave over loaded piece q of a row: fn(batch) on the elements whose
 // processed logit lies in [lo, hi] (a NaN counts as inside), in no particular
 // order. fn evaluates p exactly (some 32 instructions, in binary64), and a pass
 // wants few of the elements, so each element's test only appends it to the
 // wave's queue in LDS and fn runs on full waves of queued ones. The piece's
-// elements are all done on return.
+// elements are all done on return. Of the piece's steps st0 .. st1 - 1 are taken.
 // kWhole: with lo = -inf every element is wanted, and goes to fn without the
 // queue.
 template <int DT, int kBeside, bool kWhole, class FS, typename Fn>
 __device__ __forceinline__ void piece_pass(const Params& p, const Piece<DT>& c, const Piece<DT>& c1, int q, float lo,
-                                           float hi, uint32_t* queue, Fn fn) {
+                                           float hi, uint32_t* queue, Fn fn, int st0 = 0,
+                                           int st1 = Pass<DT, kBeside>::kSteps) {
   using B = Batch<kBeside, FS>;
   constexpr int kWords = kBeside == kAlone ? 1 : 2;
-  constexpr int kStep = kBeside == kAlone ? 4 : 2;  // elements between drains
-  constexpr int kSteps = Piece<DT>::kElems / kWave / kStep;
+  constexpr int kStep = Pass<DT, kBeside>::kStep;
   static_assert((kStep + B::kN) * kWave * kWords <= kQueue, "queue size");
   const int lane = threadIdx.x & (kWave - 1);
   const bool pen = p.use_pen != 0;
   uint32_t n = 0;  // queued (wave-uniform)
 #pragma unroll 1
-  for (int st = 0; st < kSteps; ++st) {
+  for (int st = st0; st < st1; ++st) {
     float x[kStep], x1[kStep];
     int i0;
     piece_step<DT, kStep>(p, c, c.bits, pen, q, st, x, &i0);
@@ -1710,7 +1719,7 @@ __device__ __forceinline__ void piece_pass(const Params& p, const Piece<DT>& c, 
     }
     wave_lds_fence();
     // whole batches; after the last step also the rest
-    const uint32_t most = st == kSteps - 1 ? 0u : B::kN * kWave - 1;
+    const uint32_t most = st == st1 - 1 ? 0u : B::kN * kWave - 1;
 #pragma unroll 1
     while (n > most) {
       const uint32_t take = n < static_cast<uint32_t>(B::kN * kWave) ? n : static_cast<uint32_t>(B::kN * kWave);
@@ -2072,29 +2081,46 @@ __device__ __forceinline__ bool refill_chunks(const Params& p, FS& f, int s, int
   const float lo = x_floor(K, c);
   uint32_t* q = wave_queue(f);
   // the chunks to re-read (lane l's bounds are chunk l's and chunk 64 + l's),
-  // dealt to the waves in turn
+  // dealt to the waves in turn: whole ones, or, when they are fewer than the
+  // waves, as many parts of each as give every wave one (a chunk read by one
+  // wave while the others waited took 1.5 us longer)
   uint64_t need[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int j = h * kWave + lane;
     need[h] = __ballot(j < p.nch && f.bound[s][j < p.nch ? j : 0] >= c);
   }
+  const int chunks = __builtin_popcountll(need[0]) + __builtin_popcountll(need[1]);
+  const int parts = chunks > 4 ? 1 : (chunks > 2 ? 2 : (chunks == 2 ? 4 : 8));
+  constexpr int kPer = Piece<DT>::kPerChunk;
+  constexpr int kStep = Pass<DT, kIndex>::kStep, kSteps = Pass<DT, kIndex>::kSteps;
+  static_assert(kSteps * kPer % 8 == 0 && kFNW == 8, "whole steps per part");
+  const int per_part = kSteps * kPer / parts;
   int turn = 0;
 #pragma unroll 1
   while (need[0] | need[1]) {
     const int hi = need[0] ? 0 : 1;
     const int j = hi * kWave + __builtin_ctzll(hi ? need[1] : need[0]);
     if (hi) need[1] &= need[1] - 1; else need[0] &= need[0] - 1;
-    if ((turn++ & (kFNW - 1)) != w) continue;
-    constexpr int kPer = Piece<DT>::kPerChunk;
+    const int part = (w - turn) & (kFNW - 1);
+    turn += parts;
+    if (part >= parts) continue;
     Piece<DT> cd[kPer];
-#pragma unroll
-    for (int h = 0; h < kPer; ++h) load_piece<DT>(p, rowp, bm, j * kPer + h, cd[h]);
-    const uint32_t e0 = f.cstart[s][j], e1 = e0 + f.ccount[s][j];
-    for (uint32_t e = e0 + lane; e < e1; e += kWave) f.ent[s].pbits[e] = 0u;
+    int st0[kPer], st1[kPer];  // this wave's steps of each piece
 #pragma unroll
     for (int h = 0; h < kPer; ++h) {
-      if ((j * kPer + h) * Piece<DT>::kElems >= p.vocab) break;
+      const int a = part * per_part - h * kSteps, b = a + per_part;
+      st0[h] = a < 0 ? 0 : a;
+      st1[h] = b > kSteps ? kSteps : b;
+      load_piece<DT>(p, rowp, bm, j * kPer + h, cd[h], st0[h] * kStep / Elem<DT>::kPerVec,
+                     (st1[h] * kStep + Elem<DT>::kPerVec - 1) / Elem<DT>::kPerVec);
+    }
+    if (part == 0) {
+      const uint32_t e0 = f.cstart[s][j], e1 = e0 + f.ccount[s][j];
+      for (uint32_t e = e0 + lane; e < e1; e += kWave) f.ent[s].pbits[e] = 0u;
+    }
+#pragma unroll
+    for (int h = 0; h < kPer; ++h) {
       piece_pass<DT, kIndex, false, FS>(p, cd[h], cd[h], j * kPer + h, lo, __builtin_inff(), q,
                                  [&](const Batch<kIndex, FS>& b) {
         float v[b.kN];
@@ -2103,7 +2129,7 @@ __device__ __forceinline__ bool refill_chunks(const Params& p, FS& f, int s, int
 #pragma unroll
         for (int k = 0; k < b.kN; ++k)
           list_append<true>(f, s, &f.aux[s].n, b.valid[k] && v[k] >= c, __float_as_uint(v[k]), b.beside[k]);
-      });
+      }, st0[h], st1[h]);
     }
   }
   __syncthreads();
