@@ -18,7 +18,7 @@
 // per flop, above the LDS read rate at the MFMA peak). Both operands are staged
 // through LDS in k-blocks of 64 (16-byte chunks XOR-swizzled by row) by direct
 // global-to-LDS loads (global_load_lds_dwordx4): the weight two or three blocks
-// ahead (non-temporal: read once), so that those HBM reads are in flight while
+// ahead (non-temporal, see dma16_stream), so that those HBM reads are in flight while
 // a block is multiplied and no registers hold them, the hidden rows
 // (L2-resident, re-read by every column block) one or two blocks ahead. Each
 // block ends with an explicit wait that leaves the newest loads in flight and a
@@ -51,7 +51,7 @@ constexpr int kLmLanes = 512;
 constexpr int kLmWaves = kLmLanes / 64;         // 8: 4 (rows) x 2 (columns)
 constexpr int kLmNT = 6;                       // 16-column tiles per wave
 constexpr int kLmColsPerWave = 16 * kLmNT;     // 96
-constexpr int kLmMaxRows = 320;                // rows per workgroup: 64 MT for MT = 3, 4 or 5 16-row tiles per wave
+constexpr int kLmMaxRows = 320;                // rows per workgroup at most (64 MT of them, MT = 1..5)
 constexpr int kLmBN = 2 * kLmColsPerWave;      // 192 columns per workgroup
 constexpr int kLmKB = 64;                      // k per LDS block
 constexpr int kXcds = 8;
@@ -66,7 +66,7 @@ struct LmParams {
   int64_t ws;
   int64_t M, H, V;
   int nblk;             // column blocks (ceil(V / 192))
-  int mblk;             // row blocks (ceil(M / 320))
+  int mblk;             // row blocks (ceil(M / 320); each of 64 MT rows, MT by the rows per block)
   uint64_t* keys;       // [nblk, M] partial keys
   int64_t* out;         // [M]
   void* logits;         // logits epilogue: [M, V] float32 or bf16, row stride los elements
@@ -90,9 +90,14 @@ __device__ __forceinline__ void dma16(const void* src, uint32_t lds) {
   asm volatile("global_load_lds_dwordx4 %0, off" : : "v"(src), "{m0}"(lds) : "memory");
 }
 
-// The same with the non-temporal hint, for the weight: each of its lines is
-// read once, and without the hint the 201 MB stream evicts the hidden rows
-// (1.3 MB, re-read by every column block) from L2 (C2H: 69.6 -> 66.3 us).
+// The same with the non-temporal hint, for the weight: a line is read by the
+// row blocks of one column block and then no more, while the hidden rows are
+// re-read by every column block. After other traffic (2 GB written before each
+// call; H 2048, V 49152) the hint is worth 102 -> 56 us at 65 rows, 114 -> 76
+// at 320, 165 -> 149 at 700. Calls back to back, which nothing separates and
+// which find part of the 201 MB weight in the Infinity Cache without it, take
+// 66 us with it and 61 without at 320 rows, 144 and 138 at 700; a weight that
+// does not fit there (1 GB, 1280 rows) 1100 and 1104.
 __device__ __forceinline__ void dma16_stream(const void* src, uint32_t lds) {
   asm volatile("global_load_lds_dwordx4 %0, off nt" : : "v"(src), "{m0}"(lds) : "memory");
 }
@@ -107,7 +112,7 @@ __device__ __forceinline__ int head_block() {
 // Byte offset of 16-byte chunk c of row r in an A block.
 __device__ __forceinline__ int a_off(int r, int c) { return r * kLmRowBytes + ((c ^ (r & 7)) << 4); }
 
-// More than 128 rows; a workgroup takes kBM of them.
+// More than 32 rows; a workgroup takes kBM of them.
 template <int MT, int EPI>
 __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
   constexpr int kRowsPerWave = 16 * MT;
@@ -145,7 +150,7 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
   // Direct loads: round i of wave w puts lane l's 16 bytes at LDS chunk
   // j = (8i + w) * 64 + l, i.e. row j/8 of the buffer, swizzled chunk l & 7,
   // so the lane fetches logical chunk (l & 7) ^ (row & 7) of that row. A block
-  // of hidden rows is 40 such 1 KB rounds (five per wave), one of weight rows
+  // of hidden rows is 8 MT such 1 KB rounds (MT per wave), one of weight rows
   // 24 (three per wave). Rows past the matrix are clamped into it (their
   // results are never used). Byte offsets from the block's first row.
   const uint32_t lchunk = static_cast<uint32_t>(((lane & 7) ^ ((lane >> 3) & 7)) << 4);
@@ -193,7 +198,7 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
   // is an immediate offset)
   const int fr_a = (wm * kRowsPerWave + (lane & 15)) * kLmRowBytes;
   const int fr_b = (wn * kLmColsPerWave + (lane & 15)) * kLmRowBytes;
-  // One k-block: 2 k-steps x 5 row tiles. Each tile's fragment (and each
+  // One k-block: 2 k-steps x MT row tiles. Each tile's fragment (and each
   // k-step's column fragments) is read one tile ahead, before the current
   // tile's MFMAs, so the LDS latency overlaps them; a scheduling fence after
   // each tile keeps the compiler from hoisting every read.
@@ -341,18 +346,16 @@ __global__ __launch_bounds__(kLmLanes) void lm_head_kernel(const LmParams p) {
 constexpr int kDppRowRor8 = 0x128;
 constexpr int kLrLanes = 768;
 constexpr int kLrWaves = kLrLanes / 64;  // one per 16 columns
-constexpr int kLrAhead = 4;              // k-blocks of weight in flight per wave
+constexpr int kLrAhead = 4;              // k-blocks of weight in flight per wave, and per LDS buffer of hidden rows
 static_assert(kLrWaves * 16 == kLmBN, "the same column blocks as lm_head_kernel (their keys share a layout)");
 
 template <int MT, int EPI>
 __global__ __launch_bounds__(kLrLanes) void lm_head_rows_kernel(const LmParams p) {
   constexpr int kRows = 16 * MT;
-  constexpr int kSteps = 4;                      // k-blocks per LDS buffer
   constexpr int kStepBytes = kRows * kLmRowBytes;
-  constexpr int kDeep = kLrAhead / kSteps;       // buffers of hidden rows on their way in registers
-  constexpr int kChunks = kSteps * kStepBytes / 16;
+  constexpr int kChunks = kLrAhead * kStepBytes / 16;
   constexpr int kRounds = (kChunks + kLrLanes - 1) / kLrLanes;
-  __shared__ __attribute__((aligned(16))) uint8_t abuf[2][kSteps * kStepBytes];
+  __shared__ __attribute__((aligned(16))) uint8_t abuf[2][kLrAhead * kStepBytes];
   __shared__ uint64_t keys[kRows][kLrWaves];
   const int t = threadIdx.x, lane = t & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(t / kWave);
@@ -388,7 +391,7 @@ __global__ __launch_bounds__(kLrLanes) void lm_head_rows_kernel(const LmParams p
     aoff[r] = static_cast<uint32_t>(astep[r] * kStepBytes + a_off(row, ch));
     ap[r] = p.hidden + (row < p.M ? row : p.M - 1) * p.hs * 2 + ch * 16;
   }
-  u32x4 areg[kDeep][kRounds];
+  u32x4 areg[kRounds];  // the next buffer of hidden rows on its way
   auto load_a = [&](int kb0, u32x4 (&d)[kRounds]) {  // the buffer of k-blocks kb0 .. (past the last: the last again, not used)
 #pragma unroll
     for (int r = 0; r < kRounds; ++r) {
@@ -451,15 +454,14 @@ __global__ __launch_bounds__(kLrLanes) void lm_head_rows_kernel(const LmParams p
   };
 
   // Loads return in order, so hidden rows asked for after a k-block's weight
-  // arrive after it: they go out as far ahead as the weight does (buffer q of
-  // the next group's beside k-block q * kSteps of its weight), or waiting for
-  // them would wait for all the weight under way.
+  // arrive after it: those of a group go out before its weight, a group
+  // ahead, or waiting for them would wait for all the weight under way.
   u32x4 first[kRounds];
   load_a(0, first);
 #pragma unroll
   for (int u = 0; u < kLrAhead; ++u) {
     load_b(u, b[u]);
-    if (u % kSteps == kSteps - 1) load_a(u + 1, areg[u / kSteps]);
+    if (u == kLrAhead - 1) load_a(kLrAhead, areg);
     __builtin_amdgcn_sched_barrier(0);
   }
   store_a(abuf[0], first);
@@ -471,12 +473,12 @@ __global__ __launch_bounds__(kLrLanes) void lm_head_rows_kernel(const LmParams p
   for (; kb0 + kLrAhead < nkb; kb0 += kLrAhead) {
 #pragma unroll
     for (int u = 0; u < kLrAhead; ++u) {
-      multiply(abuf[cur] + (u % kSteps) * kStepBytes, b[u]);
+      multiply(abuf[cur] + u * kStepBytes, b[u]);
       __builtin_amdgcn_sched_barrier(0);
       load_b(kb0 + u + kLrAhead, b[u]);
-      if (u % kSteps == kSteps - 1) {
-        store_a(abuf[cur ^ 1], areg[u / kSteps]);
-        load_a(kb0 + u + kLrAhead + 1, areg[u / kSteps]);
+      if (u == kLrAhead - 1) {
+        store_a(abuf[cur ^ 1], areg);
+        load_a(kb0 + 2 * kLrAhead, areg);
         meet();
         cur ^= 1;
       }
@@ -486,14 +488,7 @@ __global__ __launch_bounds__(kLrLanes) void lm_head_rows_kernel(const LmParams p
   // the last group (1 .. kLrAhead k-blocks)
 #pragma unroll
   for (int u = 0; u < kLrAhead; ++u) {
-    if (kb0 + u < nkb) {
-      multiply(abuf[cur] + (u % kSteps) * kStepBytes, b[u]);
-      if (u % kSteps == kSteps - 1 && kb0 + u + 1 < nkb) {
-        store_a(abuf[cur ^ 1], areg[u / kSteps]);
-        meet();
-        cur ^= 1;
-      }
-    }
+    if (kb0 + u < nkb) multiply(abuf[cur] + u * kStepBytes, b[u]);
   }
 
   // accumulator i of row tile mt is row mt * 16 + (lane / 16) * 4 + i
@@ -665,7 +660,7 @@ int lm_head_launch(const char* what, const void* hidden, int64_t hidden_stride, 
   const int64_t nblk = (vocab + kLmBN - 1) / kLmBN;
   const int64_t mblk = (rows + kLmMaxRows - 1) / kLmMaxRows;
   if (mblk > 65535) return fail(LS_ERR_VALUE, w + ": too many rows");
-  // (their keys or logits would fill hundreds of GB)
+  // (their keys or logits would fill terabytes)
   if (launched_cols(nblk, mblk) * mblk > 0x7fffffffLL - (1LL << kGridXLog2))
     return fail(LS_ERR_VALUE, w + ": rows x vocab too large");
   if (epi == kLmKeys && (workspace == nullptr || ws_bytes < ls_lm_head_argmax_workspace(rows, vocab)))
