@@ -15,9 +15,10 @@ cutoff among the candidates and takes one of these paths:
               their {p >= cutoff} replaces their candidates (fits in 2048
               entries), then the cutoff is selected again;
   slow_list   the candidates hold less than top_p, or the refill overflows:
-              the whole row is selected by passes over it, and its support
-              (<= 2048 elements) is kept in the entries;
-  slow_dense  as slow_list with a larger support: the draws pass over the row.
+              the whole row is selected by passes over it, and so are the
+              draws made; its support has at most 2048 elements;
+  slow_dense  as slow_list with a larger support (with top-k it does not fit
+              the list that the k-th largest is counted in).
 
 The paths must give identical results; the oracle computes the result
 directly. This restates the candidate rule for rows without a penalty (x in

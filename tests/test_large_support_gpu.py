@@ -33,6 +33,8 @@ BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
     (2, 1, 32000, F32, 1.0, 0.99, 3000, 1.0),  # top-k beyond the candidates, both whole-row selects
     (2, 1, 49152, F32, 1.0, 0.2, 2500, 1.0),   # top-p inside the candidates, top-k beyond them
     (130, 1, 8192, BF16, 1.0, 0.97, 600, 1.1),
+    (130, 1, 8192, F32, 1.0, 1.0, 0, 1.0),     # unfiltered rows, two workgroups per CU
+    (130, 1, 2056, BF16, 1.0, 1.0, 0, 1.2),
 ])
 def test_spec_verify_large_supports(gpu, batch, k, vocab, dtype, t, top_p, top_k, penalty):
     pen = penalty != 1.0

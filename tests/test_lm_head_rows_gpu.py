@@ -31,6 +31,27 @@ def test_lm_head_rows(gpu, rows, hidden_size, vocab):
     assert bool((out[rows] == 7.0).all()) and bool((out[:, vocab:] == 7.0).all())
 
 
+@pytest.mark.parametrize("hidden_size", [192, 896, 1664])
+@pytest.mark.parametrize("rows", [20, 33, 96, 128, 192, 256, 321])
+def test_lm_head_bf16_logits_and_whole_ring_turns(gpu, rows, hidden_size):
+    """bf16 logits of every tile height, at hidden sizes below, past and at twice
+    the 12 k-blocks that the tallest unrolled loop takes per turn (3, 14, 26)."""
+    vocab = 451
+    hidden, weight = make(rows, hidden_size, vocab, rows + hidden_size)
+    announce(f"lm_head bf16 logits M={rows} H={hidden_size} V={vocab}")
+    h, w = hidden.to(gpu), weight.to(gpu)
+    out = torch.full((rows + 1, vocab + 13), 7.0, dtype=torch.bfloat16, device=gpu)
+    b16 = verify.lm_head_logits(h, w, out=out[:rows, :vocab])
+    f32 = verify.lm_head_logits(h, w)
+    ids = verify.lm_head_argmax(h, w)
+    torch.cuda.synchronize()
+    logits, bound = reference(hidden, weight)
+    assert bool(((f32.double().cpu() - torch.from_numpy(logits)).abs() <= torch.as_tensor(bound)).all())
+    assert torch.equal(b16, f32.to(torch.bfloat16))  # the same sums, rounded once
+    assert torch.equal(f32.argmax(-1), ids)
+    assert bool((out[rows] == 7.0).all()) and bool((out[:, vocab:] == 7.0).all())
+
+
 def test_lm_head_more_workgroups_than_one_launch_dimension(gpu):
     """10,485,800 rows at 256 column blocks: 2^23 workgroups of 512 lanes and more
     than 2^32 lanes. The rows repeat 97 others, whose period meets every place of a
