@@ -1539,9 +1539,6 @@ __device__ __forceinline__ void select_entries(FS& f, uint32_t mask, const uint6
 // ---------------------------------------------------------------------------
 // Whole-row passes: rows whose support is not among their candidates
 // ---------------------------------------------------------------------------
-// They are inlined into the finaliser, and the branches to them say that they
-// are the rare case, which keeps their code out of the way of the common one's:
-// B 64, k 2, V 49152 f32, top-p 0.7, 35.0 us a call without, 34.5 with.
 constexpr int kQueue = kHash / kFNW;  // words of LDS (the draft hash's) a wave queues logits in
 
 // Logits that bracket an element's p without forming it. p = RN(e / S) with
@@ -2185,7 +2182,7 @@ __device__ __forceinline__ void resolve_rows(const Params& p, FS& f, const int (
       late |= 1u << s;
     }
   }
-  if (__builtin_expect(!(late | whole), 1)) return;
+  if (!(late | whole)) return;
   __syncthreads();  // every read of the rows' state above precedes the stores
   if (threadIdx.x == 0) {
 #pragma unroll
@@ -2197,7 +2194,7 @@ __device__ __forceinline__ void resolve_rows(const Params& p, FS& f, const int (
   const float g1 = uniform<FS>(ok[1] ? cut[1] : cutoff_guess(p, thr[1]));
 #pragma unroll 1
   for (int s = 0; s < 2; ++s) {
-    if (__builtin_expect(!((whole >> s) & 1u), 1)) continue;
+    if (!((whole >> s) & 1u)) continue;
     const int row = s == 0 ? rows[0] : rows[1];
     const RowK Ks = s == 0 ? K[0] : K[1];
     const uint64_t th = s == 0 ? thr[0] : thr[1];
@@ -2337,7 +2334,7 @@ __device__ __forceinline__ void resolve_top_k(const Params& p, FS& f, const int 
   for (int s = 0; s < 2; ++s) {
     if (((mask >> s) & 1u) && !(((kmask >> s) & 1u) && mass[s] < thr[s])) pmask |= 1u << s;
   }
-  if (__builtin_expect(pmask != 0, 0)) resolve_rows<DT>(p, f, rows, K, pmask, thr, eb, ew, false);
+  if (pmask) resolve_rows<DT>(p, f, rows, K, pmask, thr, eb, ew, false);
   uint32_t store = 0, emask = 0, whole = 0;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
@@ -2383,7 +2380,7 @@ __device__ __forceinline__ void resolve_top_k(const Params& p, FS& f, const int 
   }
 #pragma unroll 1
   for (int s = 0; s < 2; ++s) {
-    if (__builtin_expect(!((whole >> s) & 1u), 1)) continue;
+    if (!((whole >> s) & 1u)) continue;
     // the k-th largest of the whole row by passes over it
     const int row = s == 0 ? rows[0] : rows[1];
     const RowK Ks = s == 0 ? K[0] : K[1];
@@ -2599,7 +2596,7 @@ template <int DT, class FS>
 __device__ __forceinline__ float q_at(const Params& p, const FS& f, const RowK& K1, int row1, uint32_t x) {
   const RowAux& a = f.aux[1];
   if (a.flags & kRowEmpty) return 0.0f;
-  if (__builtin_expect((a.flags & kRowList) != 0, 1)) {
+  if (a.flags & kRowList) {
     // every draft element with q >= its cutoff is an entry
     const uint32_t e = hash_find(f, x);
     return e == kNone ? 0.0f : filtered_of(a, __uint_as_float(f.ent[1].pbits[e]));
@@ -2616,7 +2613,7 @@ __device__ __forceinline__ float support_floor(const RowAux& a, const RowK& K) {
 template <int DT, class FS>
 __device__ __forceinline__ int64_t draw_target(const Params& p, FS& f, int row0, const RowK& K0, float u) {
   const RowAux& a = f.aux[0];
-  if (__builtin_expect((a.flags & kRowList) != 0, 1)) {
+  if (a.flags & kRowList) {
     uint64_t wl[kEPT];
     const uint32_t n = a.n;
 #pragma unroll
@@ -2637,7 +2634,7 @@ __device__ __forceinline__ int64_t draw_residual(const Params& p, FS& f, int row
                                  float u) {
   const int t = thread_index<FS>();
   const RowAux& a = f.aux[0];
-  if (__builtin_expect((a.flags & kRowList) != 0, 1)) {
+  if (a.flags & kRowList) {
     const uint32_t n = a.n;
     const RowAux& a1 = f.aux[1];
     // P and d = max(P - Q, 0) at the entries t + kFW q (every wave takes a
