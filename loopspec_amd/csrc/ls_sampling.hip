@@ -1056,7 +1056,10 @@ struct FinShT {
 static_assert(sizeof(FinShT<10>) <= 80 * 1024, "two finaliser workgroups per CU");
 
 // With two finaliser workgroups per CU (128 registers) the whole-row passes need
-// every vector register, and what the set-up keeps for them would spill there.
+// every vector register, and much of what the set-up keeps for them would spill
+// there (24 to 32 bytes per lane still do; the finaliser had no scratch before it
+// had these passes, and B 128, k 2, V 49152 f32, top-p 0.7 took 51.3 us a call
+// then, 51.0 with them).
 // uniform: a value every lane holds alike, in scalar registers. thread_index: the
 // thread's index, opaque to the compiler, so that addresses formed from it are
 // formed again where they are used. Where one workgroup has the CU both are left
@@ -3309,7 +3312,11 @@ int ls_filter_logits(const void* logits, int64_t row_stride, int dtype, int64_t 
               (!filtered_out || (aligned16(filtered_out) && filtered_stride % 4 == 0));
   // Without the unfiltered rows, a filtered row is zeros but for its support,
   // which the finaliser holds: no second pass over the logits (64 rows, V 49152
-  // f32, top-p 0.7: 27.0 -> 23.3 us a call; 200 rows, V 128256 bf16: 106 -> 57).
+  // f32, T 1, top-p 0.7: 23.5 us a call with dense_kernel writing every row, 21.3
+  // so; 200 rows, V 128256 bf16 128.5 and 120.6). The rule cannot know the
+  // supports: a row whose support is not in the finaliser's list is written
+  // twice, the zeros for nothing (top-p 0.95: 50.9 and 53.7; 115.4 and 129.2;
+  // unfiltered rows, by a top_p_rows of 1, 18.5 and 21.0).
   // Not where the output overlaps the logits, which the finaliser may read again.
   auto disjoint = [&](const void* x, int64_t xs, int64_t xb, const void* y, int64_t ys, int64_t yb) {
     const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
